@@ -113,6 +113,28 @@ def test_emccd_parity_common_total_and_long_supports(gpu):
         assert numpy.array_equal(adc.cpu().numpy().reshape(E.shape), ref_adc)
 
 
+@pytest.mark.parametrize('emgain', [1, 8, 9, 63, 64, 65, 128, 129, 192, 300, 577, 1000])
+def test_emccd_parity_gains(gpu, emgain):
+    """Draws equal the oracle's at the edges of the run lengths (direct terms up
+    to a gain of 8, pieces of 64 terms above 128, eight pieces a pass), for
+    supports that start at 0 and beyond it and uniforms at both ends.  Equality
+    is the expected outcome: the cumulative masses of the two agree to ~1e-14,
+    so a draw differs only if one of these uniforms lies that close to one of
+    at most ~1e5 steps."""
+    rng = numpy.random.RandomState(emgain)
+    E = numpy.concatenate([[0.0092, 1e-9, 0.4, 3.0, 11.0, 37.0, 43.5, 44.5, 90.0, 333.3, 705.0],
+                           rng.uniform(0.0, 30.0, 13)]).reshape(4, 6)
+    u = rng.random_sample(E.size)
+    u[[2, 3, 4]] = 0.0, 1.0 - 2.0 ** -30, 1e-12
+    p = oracle_params({'detector': {'image_size': [4, 6], 'emgain': emgain}})
+    noise = numpy.zeros(E.shape)
+    ref_adc, ref_S = _oracle(p, E, noise, u)
+    adc, S, status = _gpu_parity(gpu, E, noise, u, _det_params(p))
+    assert status == 0
+    assert numpy.array_equal(S, ref_S)
+    assert numpy.array_equal(adc, ref_adc)
+
+
 def test_emccd_parity_fpn_maps(gpu):
     rng = numpy.random.RandomState(3)
     p = oracle_params({'detector': {'image_size': [16, 16]},
