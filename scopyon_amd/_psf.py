@@ -127,8 +127,8 @@ class PSFTables:
             j0w = _device.ARENA.typed('psf_j0', self.nr * 100, torch.float64, self.device)
             _lib.call('smx_psf_radial_born_wolf', depths.data_ptr(), nz, self.nr, RES, self.alpha,
                       self.gamma, self.scale, j0w.data_ptr(), radial.data_ptr(), st)
-        # build in batches so the row-sum scratch stays bounded (~64 MB per table)
-        batch = 8
+        # build in batches so the scratch stays bounded (~1 MB per table)
+        batch = 64
         for s in range(0, nz, batch):
             m = min(batch, nz - s)
             ws = _device.ARENA.get('psf_satws', lib.smx_psf_sat_workspace_bytes(self.nr, m),

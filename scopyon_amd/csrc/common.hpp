@@ -199,30 +199,22 @@ __device__ inline float dpp_f32(float v) {
 }
 
 // Summed-area-table index for a (side x side) corner grid stored either
-// row-major (period == 1) or phase-major with the given period: corners whose
-// row/column indices share residues mod `period` are contiguous, so one
-// emitter's regular pixel-boundary grid reads a compact block.
+// row-major (period == 1) or phase-major with the given period: on each axis
+// corner a takes place (a mod period) g + a / period, so corners a pixel
+// apart are neighbours and one emitter's row of pixel boundaries is one
+// contiguous run.  Whole rows stay contiguous, which is how the tables are
+// built and read.
 struct SatLayout {
     int side;     // corner indices 0..side-1 on each axis (table side + 1)
     int period;   // >= 1
     int g;        // ceil(side / period)
-    SMX_HD size_t index(int a, int b) const {
-        if (period == 1) return (size_t)a * side + b;
-        int pa = a % period, pb = b % period;
-        return ((size_t)(pa * period + pb) * g + (a / period)) * g + (b / period);
-    }
+    int width;    // places per axis: period * g (side when period == 1)
+    SMX_HD int place(int a) const { return period == 1 ? a : (a % period) * g + a / period; }
     // index(a, b) == row_part(a) + col_part(b)
-    SMX_HD size_t row_part(int a) const {
-        if (period == 1) return (size_t)a * side;
-        return (size_t)(a % period) * period * g * g + (size_t)(a / period) * g;
-    }
-    SMX_HD size_t col_part(int b) const {
-        if (period == 1) return (size_t)b;
-        return (size_t)(b % period) * g * g + (size_t)(b / period);
-    }
-    SMX_HD size_t elems() const {
-        return period == 1 ? (size_t)side * side : (size_t)period * period * g * g;
-    }
+    SMX_HD size_t row_part(int a) const { return (size_t)place(a) * width; }
+    SMX_HD size_t col_part(int b) const { return (size_t)place(b); }
+    SMX_HD size_t index(int a, int b) const { return row_part(a) + col_part(b); }
+    SMX_HD size_t elems() const { return (size_t)width * width; }
 };
 
 SMX_HD SatLayout make_sat_layout(int side, int period) {
@@ -230,6 +222,7 @@ SMX_HD SatLayout make_sat_layout(int side, int period) {
     L.side = side;
     L.period = period < 1 ? 1 : period;
     L.g = (side + L.period - 1) / L.period;
+    L.width = L.period == 1 ? side : L.period * L.g;
     return L;
 }
 
