@@ -61,6 +61,18 @@ size_t smx_psf_sat_workspace_bytes(int nr, int nz);
 int smx_psf_sat_build(const double* radial, int nz, int nr, double res, int period,
                       double* workspace, double* sat, hipStream_t stream);
 
+/* The same tables in the sorted layout, for pixels that are not an integer
+ * number of cells (ratio = pixel length / res): places[b] (2 nr ints, written
+ * to host memory by smx_sat_sorted_places; the build and the splat take a
+ * device copy) orders the corners of an axis so that any emitter's pixel
+ * boundaries are one run.  smx_psf_sat_sorted_elems(nr) doubles per table
+ * (0: too wide for this layout, 2 nr - 1 > 4096); workspace as for
+ * smx_psf_sat_build. */
+size_t smx_psf_sat_sorted_elems(int nr);
+int smx_sat_sorted_places(int nr, double ratio, int* places /* host */);
+int smx_psf_sat_build_sorted(const double* radial, int nz, int nr, double res, const int* places,
+                             double* workspace, double* sat, hipStream_t stream);
+
 /* Radial x depth lookup-table PSF (smx_lut_t, scopyon_hip_types.h): per
  * depth slice z, the float32 pixel integrals K[qu][qv][du][dv]
  * (smx_lut_table_elems floats) of the cartesian kernel built from the
@@ -174,6 +186,11 @@ int smx_splat_accumulate(int n, const double* u, const double* v, const double* 
  * workload and keeps the fastest.  No reference counterpart (the reference
  * loops over emitters on the whole frame, _epifm.py:215-282). */
 #define SMX_TILE_Q32 0x100
+/* k_format of the splat calls when `sat` holds sorted tables
+ * (smx_psf_sat_build_sorted): no phase table, K is the device copy of their
+ * places; every FOV's pixel length over res is the ratio they were made for
+ * (another is correct, only slower).  Not with a detector epilogue. */
+#define SMX_K_PLACES 3
 /* Or-ed into the tile side: this workspace was binned before by a call with
  * the same FOV layout, tile side, emitter count and list capacity, so its
  * tile counters are back at zero (the fill counts them down) and its tile ->

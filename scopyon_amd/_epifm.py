@@ -287,11 +287,11 @@ class Splatter:
         cap = max(1, n * tiles_per_emitter(self.c.pixel_length, t.ntab))
         nbytes = lib.smx_splat_workspace_bytes(n, n_tiles, cap)
         ws = _device.ARENA.get('splat_ws', nbytes, self.device)
-        K = t.K if (t.use_phase and self.use_phase) else None
+        sat, stride, K, kf = t.splat_tables(t.K if (t.use_phase and self.use_phase) else None)
         _lib.call('smx_splat_expected', n, _device.ptr(u), _device.ptr(v), _device.ptr(w),
                   _device.ptr(key), _device.ptr(fov_id), fovs_dev.data_ptr(), nfov, n_tiles,
-                  t.sat.data_ptr(), t.sat_elems, len(t.slot_of), t.ntab, t.period, RES, RES * RES,
-                  cap, 1 if accumulate else 0, _device.ptr(K), 0, t.m, out.data_ptr(),
+                  sat, stride, len(t.slot_of), t.ntab, t.period, RES, RES * RES,
+                  cap, 1 if accumulate else 0, K, kf, t.m, out.data_ptr(),
                   ws.data_ptr(), ws.numel(), self.status.data_ptr(), _device.stream())
 
 

@@ -70,6 +70,9 @@ SIGNATURES = {
     'smx_psf_sat_elems': (c_size_t, [c_int, c_int]),
     'smx_psf_sat_workspace_bytes': (c_size_t, [c_int, c_int]),
     'smx_psf_sat_build': (c_int, [P, c_int, c_int, c_double, c_int, P, P, P]),
+    'smx_psf_sat_sorted_elems': (c_size_t, [c_int]),
+    'smx_sat_sorted_places': (c_int, [c_int, c_double, P]),
+    'smx_psf_sat_build_sorted': (c_int, [P, c_int, c_int, c_double, P, P, P, P]),
     'smx_emitter_weights': (c_int, [c_int, P, P, ctypes.POINTER(WeightParamsT), c_double, P, P,
                                     P, c_int, P, P, P, P]),
     'smx_splat_tiles': (c_int, [ctypes.POINTER(FovT), c_int]),

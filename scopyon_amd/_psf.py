@@ -74,12 +74,24 @@ class PSFTables:
         self.cutoff_index = self.n_keys - 1
         self.slot_of = {}
         self.capacity = 0
-        self.sat = None
+        self._sat = None
+        self._plain = None
         # phase tables (integer pixel/cell ratio only): footprint pixels per axis
         self.m = int(math.ceil(RES * (self.ntab - 1) / pixel_length)) + 2 if pixel_length else 0
         self.use_phase = bool(pixel_length) and sat_period(pixel_length) > 1
         self.k_elems = (int(_lib.lib().smx_phase_table_elems(self.period, self.m))
                         if self.use_phase else 0)
+        # pixels that are not whole cells: tables in the sorted layout, whose
+        # places the splat takes in place of a phase table
+        self.places = None
+        self.store_elems = self.sat_elems
+        sorted_elems = int(_lib.lib().smx_psf_sat_sorted_elems(self.nr))
+        if not self.use_phase and self.period > 1 and sorted_elems:
+            places = numpy.empty(2 * self.nr, dtype=numpy.int32)
+            _lib.call('smx_sat_sorted_places', self.nr, float(pixel_length / RES),
+                      places.ctypes.data)
+            self.places = _device.upload(places, dtype=torch.int32, device=self.device)
+            self.store_elems = sorted_elems
         self.K = None
         self._K32 = None
         self._Kfold = None
@@ -96,15 +108,65 @@ class PSFTables:
         if need <= self.capacity:
             return
         cap = max(need, 2 * self.capacity, 1)
-        new = torch.empty((cap, self.sat_elems), dtype=torch.float64, device=self.device)
-        if self.sat is not None and self.capacity:
-            new[: self.capacity].copy_(self.sat[: self.capacity])
+        new = torch.empty((cap, self.store_elems), dtype=torch.float64, device=self.device)
+        if self._sat is not None and self.capacity:
+            new[: self.capacity].copy_(self._sat[: self.capacity])
         if self.use_phase:
             newk = torch.empty((cap, self.k_elems), dtype=torch.float64, device=self.device)
             if self.K is not None and self.capacity:
                 newk[: self.capacity].copy_(self.K[: self.capacity])
             self.K = newk
-        self.sat, self.capacity = new, cap
+        self._sat, self.capacity = new, cap
+
+    def _profiles(self, keys):
+        """Radial profiles of the depth keys (one for the Gaussian PSF)."""
+        nz = len(keys)
+        radial = torch.empty((nz, self.nr), dtype=torch.float64, device=self.device)
+        if self.gaussian:
+            _lib.call('smx_psf_radial_gaussian', self.nr, RES, self.radial_width,
+                      radial.data_ptr(), _device.stream())
+        else:
+            depths = _device.upload(numpy.array([self._depth_of(k) for k in keys]),
+                                    device=self.device)
+            j0w = _device.ARENA.typed('psf_j0', self.nr * 100, torch.float64, self.device)
+            _lib.call('smx_psf_radial_born_wolf', depths.data_ptr(), nz, self.nr, RES, self.alpha,
+                      self.gamma, self.scale, j0w.data_ptr(), radial.data_ptr(), _device.stream())
+        return radial
+
+    def _build(self, radial, out, places):
+        """Summed-area tables of the profiles into out (nz, elems)."""
+        # in batches so the scratch stays bounded (~1 MB per table)
+        batch, nz = 64, radial.shape[0]
+        for s in range(0, nz, batch):
+            m = min(batch, nz - s)
+            ws = _device.ARENA.get('psf_satws', _lib.lib().smx_psf_sat_workspace_bytes(self.nr, m),
+                                   self.device)
+            if places is None:
+                _lib.call('smx_psf_sat_build', radial[s:s + m].data_ptr(), m, self.nr, RES,
+                          self.period, ws.data_ptr(), out[s].data_ptr(), _device.stream())
+            else:
+                _lib.call('smx_psf_sat_build_sorted', radial[s:s + m].data_ptr(), m, self.nr, RES,
+                          places.data_ptr(), ws.data_ptr(), out[s].data_ptr(), _device.stream())
+
+    @property
+    def sat(self):
+        """The tables in the layout of `period` (smx_psf_sat_build).  Where the
+        splat reads sorted tables these are a copy built on demand."""
+        if self.places is None:
+            return self._sat
+        keys = sorted(self.slot_of, key=self.slot_of.get)
+        if keys and (self._plain is None or len(self._plain) != len(keys)):
+            self._plain = torch.empty((len(keys), self.sat_elems), dtype=torch.float64,
+                                      device=self.device)
+            self._build(self._profiles(keys), self._plain, None)
+        return self._plain
+
+    def splat_tables(self, K=None, k_format=0):
+        """(tables, doubles per table, K, k_format) of the splat calls: the phase
+        table K, or the places of sorted tables."""
+        if self.places is not None:
+            return self._sat.data_ptr(), self.store_elems, self.places.data_ptr(), 3
+        return self._sat.data_ptr(), self.sat_elems, _device.ptr(K), k_format
 
     def ensure(self, keys):
         """Build the tables for every key in ``keys`` not built yet."""
@@ -117,26 +179,10 @@ class PSFTables:
         self._grow(base + len(missing))
         lib, st = _lib.lib(), _device.stream()
         nz = len(missing)
-        radial = torch.empty((nz, self.nr), dtype=torch.float64, device=self.device)
-        if self.gaussian:
-            _lib.call('smx_psf_radial_gaussian', self.nr, RES, self.radial_width,
-                      radial.data_ptr(), st)
-        else:
-            depths = _device.upload(numpy.array([self._depth_of(k) for k in missing]),
-                                    device=self.device)
-            j0w = _device.ARENA.typed('psf_j0', self.nr * 100, torch.float64, self.device)
-            _lib.call('smx_psf_radial_born_wolf', depths.data_ptr(), nz, self.nr, RES, self.alpha,
-                      self.gamma, self.scale, j0w.data_ptr(), radial.data_ptr(), st)
-        # build in batches so the scratch stays bounded (~1 MB per table)
-        batch = 64
-        for s in range(0, nz, batch):
-            m = min(batch, nz - s)
-            ws = _device.ARENA.get('psf_satws', lib.smx_psf_sat_workspace_bytes(self.nr, m),
-                                   self.device)
-            _lib.call('smx_psf_sat_build', radial[s:s + m].data_ptr(), m, self.nr, RES,
-                      self.period, ws.data_ptr(), self.sat[base + s].data_ptr(), st)
+        radial = self._profiles(missing)
+        self._build(radial, self._sat[base:base + nz], self.places)
         if self.use_phase:
-            _lib.call('smx_phase_table_build', self.sat[base].data_ptr(), self.sat_elems, nz,
+            _lib.call('smx_phase_table_build', self._sat[base].data_ptr(), self.sat_elems, nz,
                       self.ntab, self.period, self.m, RES * RES, self.K[base].data_ptr(), st)
         for i, k in enumerate(missing):
             self.slot_of[k] = base + i

@@ -321,11 +321,12 @@ class BatchedSimulator:
                       stages[entry], self._tile_arg())
             self._warm |= bool(stages[entry] & 1)
             return
+        sat, stride, K, kf = t.splat_tables(self.Ktab, self.k_format)
         _lib.call(entry + '_ts', self.n, self.u.data_ptr(), self.v.data_ptr(),
                   self.w.data_ptr(), self.key.data_ptr(), self.fov_id.data_ptr(),
-                  self.fovs_dev.data_ptr(), self.nfov, self.n_tiles, t.sat.data_ptr(),
-                  t.sat_elems, len(t.slot_of), t.ntab, t.period, 1e-9, 1e-18, self.capacity, 0,
-                  _device.ptr(self.Ktab), self.k_format, t.m, self.photons.data_ptr(),
+                  self.fovs_dev.data_ptr(), self.nfov, self.n_tiles, sat,
+                  stride, len(t.slot_of), t.ntab, t.period, 1e-9, 1e-18, self.capacity, 0,
+                  K, kf, t.m, self.photons.data_ptr(),
                   self.ws.data_ptr(), self.ws.numel(), self.splatter.status.data_ptr(),
                   _device.stream(), self._tile_arg())
         self._warm |= entry != 'smx_splat_accumulate'
@@ -360,10 +361,11 @@ class BatchedSimulator:
                       self.adc.data_ptr(), f32, stages[entry], self._tile_arg())
             self._warm |= bool(stages[entry] & 1)
             return
+        sat, stride, K, kf = t.splat_tables(self.Ktab, self.k_format)
         _lib.call(entry, self.n, self.u.data_ptr(), self.v.data_ptr(), self.w.data_ptr(),
                   self.key.data_ptr(), self.fov_id.data_ptr(), self.fovs_dev.data_ptr(),
-                  self.nfov, self.n_tiles, t.sat.data_ptr(), t.sat_elems, len(t.slot_of), t.ntab,
-                  t.period, 1e-9, 1e-18, self.capacity, 0, _device.ptr(self.Ktab), self.k_format,
+                  self.nfov, self.n_tiles, sat, stride, len(t.slot_of), t.ntab,
+                  t.period, 1e-9, 1e-18, self.capacity, 0, K, kf,
                   t.m, out, self.ws.data_ptr(), self.ws.numel(),
                   self.splatter.status.data_ptr(), _device.stream(), _device.ptr(self.gain_map),
                   _device.ptr(self.offset_map), self.det, self.seed, 0, 0,

@@ -226,6 +226,16 @@ SMX_HD SatLayout make_sat_layout(int side, int period) {
     return L;
 }
 
+// Sorted layout of a summed-area table whose pixels are `ratio` cells long, not
+// an integer: an emitter's corners along an axis are the cells ceil(c + ratio
+// k), k = 0, 1, ...: exactly those with c <= b - ratio floor(b / ratio) < c + 1
+// for the k they fall to.  Ordered by that phase b - ratio floor(b / ratio)
+// the corners of every possible footprint are one run of the axis.  A table is
+// side^2 corners, places[a] * side + places[b], then side zeros (corner column
+// 0) and side values of the last corner column, both in row places.
+constexpr int SAT_SORTED_MAX = 4096;   // widest table (cells) of this layout
+SMX_HD size_t sat_sorted_elems(int side) { return (size_t)side * (side + 2); }
+
 // Symmetry of the phase tables.  Along one axis an emitter of phase ph
 // (0 <= ph < P) has cell boundaries 0, ph+1, ph+1+P, ... clamped to ntab, so
 // its pixel d covers cells [edge(d), edge(d+1)) and there are

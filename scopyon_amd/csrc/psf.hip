@@ -7,6 +7,10 @@
 // from the radial profile on the fly (same interpolation as interp1d).
 #include "common.hpp"
 
+#include <algorithm>
+#include <utility>
+#include <vector>
+
 namespace {
 
 constexpr int kRho = 100;   // _epifm.py:191
@@ -100,6 +104,7 @@ __device__ inline double interp_radial(const double* __restrict__ prof, int nr, 
 // columns, 50 us so; 117 tables 14.5 ms before, 1.4 ms so.
 constexpr int kCols = 4;              // columns per thread
 constexpr int kSatMax = 1024 * kCols; // widest table of this form
+static_assert(kSatMax == smx::SAT_SORTED_MAX, "sorted tables are built by this form only");
 
 // Interval k and offset into it of the cell at (X, Y) on the radial grid
 // (scipy interp1d 'linear': the interval [x_{k-1}, x_k] with x_{k-1} < R <= x_k,
@@ -200,8 +205,12 @@ __global__ void __launch_bounds__(1024) sat_rows_kernel(int nr, int nz, double r
                                                         const double* __restrict__ prof, int ntab,
                                                         int seg, int nseg,
                                                         const double* __restrict__ sums,
-                                                        smx::SatLayout L, size_t sat_stride,
+                                                        smx::SatLayout L,
+                                                        const int* __restrict__ places,
+                                                        size_t sat_stride,
                                                         double* __restrict__ sat) {
+    // sorted layout (smx::SAT_SORTED_MAX): the axis order comes from `places`
+    auto place_of = [&](int a) { return places ? places[a] : L.place(a); };
     extern __shared__ __align__(16) double2 s_prof[];
     double* const s_wave = (double*)(s_prof + ZB * nr);  // wave totals
     double* const s_row = s_wave + 16;                   // one row in layout order
@@ -219,7 +228,7 @@ __global__ void __launch_bounds__(1024) sat_rows_kernel(int nr, int nz, double r
         const int col = t * kCols + j;
         const double X = (double)(col - (nr - 1)) * res;
         X2[j] = X * X;
-        place[j] = L.place(min(col + 1, ntab));
+        place[j] = place_of(min(col + 1, ntab));
 #pragma unroll
         for (int z = 0; z < ZB; ++z)
             C[z][j] = col < ntab && z0 + z < nz
@@ -229,13 +238,19 @@ __global__ void __launch_bounds__(1024) sat_rows_kernel(int nr, int nz, double r
     __syncthreads();
     if (blockIdx.x == 0) {
         for (int z = 0; z < ZB && z0 + z < nz; ++z) {
-            double* row0 = sat + (size_t)(z0 + z) * sat_stride + L.row_part(0);
+            double* T = sat + (size_t)(z0 + z) * sat_stride;
+            double* row0 = T + (size_t)place_of(0) * L.width;
             for (int i = t; i < L.width; i += blockDim.x) row0[i] = 0.0;
+            if (places) {   // the zeros, and row 0 of the last column
+                for (int i = t; i < L.width; i += blockDim.x) T[(size_t)L.width * L.width + i] = 0.0;
+                if (t == 0) T[(size_t)L.width * (L.width + 1) + place_of(0)] = 0.0;
+            }
         }
     }
     const int r0 = blockIdx.x * seg, r1 = min(r0 + seg, ntab);
     for (int row = r0; row < r1; ++row) {
         const double Y = (double)(row - (nr - 1)) * res, Y2 = Y * Y;
+        const int prow = place_of(row + 1);
 #pragma unroll
         for (int j = 0; j < kCols; ++j) {
             double off;
@@ -271,12 +286,19 @@ __global__ void __launch_bounds__(1024) sat_rows_kernel(int nr, int nz, double r
             for (int w = 0; w < waves; ++w)
                 if (w < wave) before += s_wave[w];
             base += before;
-            double* out = sat + (size_t)(z0 + z) * sat_stride + L.row_part(row + 1);
+            double* out = sat + (size_t)(z0 + z) * sat_stride + (size_t)prow * L.width;
+            if (places && t == (ntab - 1) / kCols) {   // the row's last corner
+                const int j = (ntab - 1) % kCols;
+                double c = 0.0;
+#pragma unroll
+                for (int y = 0; y < kCols; ++y) c = y == j ? base + run[y] : c;
+                sat[(size_t)(z0 + z) * sat_stride + (size_t)L.width * (L.width + 1) + prow] = c;
+            }
             double* to = STAGED ? s_row : out;
 #pragma unroll
             for (int j = 0; j < kCols; ++j)
                 if (t * kCols + j < ntab) to[place[j]] = base + run[j];
-            if (!STAGED && t == 0) out[L.place(0)] = 0.0;
+            if (!STAGED && t == 0) out[place_of(0)] = 0.0;
             __syncthreads();
             if (STAGED)
                 for (int i = t; i < L.width; i += blockDim.x)
@@ -360,7 +382,7 @@ int sat_segment_rows(int nz) { return nz <= 4 ? 8 : 32; }
 
 template <int ZB, bool STAGED>
 int sat_build(const double* radial, int nz, int nr, double res, int ntab, smx::SatLayout L,
-              double* sums, double* sat, hipStream_t stream) {
+              const int* places, size_t stride, double* sums, double* sat, hipStream_t stream) {
     const int seg = sat_segment_rows(nz), nseg = (ntab + seg - 1) / seg, nzb = (nz + ZB - 1) / ZB;
     const size_t lds = sizeof(double2) * ZB * (size_t)nr;
     // every block computes the slopes of its profiles, so a block takes whole
@@ -379,9 +401,22 @@ int sat_build(const double* radial, int nz, int nr, double res, int ntab, smx::S
     const int threads = ((ntab + kCols - 1) / kCols + 63) / 64 * 64;
     hipLaunchKernelGGL((sat_rows_kernel<ZB, STAGED>), dim3(nseg, nzb), dim3(threads),
                        lds + sizeof(double) * (size_t)(16 + (STAGED ? L.width : 0)), stream, nr,
-                       nz, res, radial, ntab, seg, nseg, sums, L, L.elems(), sat);
+                       nz, res, radial, ntab, seg, nseg, sums, L, places, stride, sat);
     SMX_CHECK_LAUNCH("sat_rows_kernel");
     return SMX_OK;
+}
+
+int sat_build_any(const double* radial, int nz, int nr, double res, int ntab, smx::SatLayout L,
+                  const int* places, size_t stride, double* sums, double* sat, hipStream_t stream) {
+    // two depths' profiles a block and the staged row while 64 KB of LDS
+    // hold them (they do up to 1 um radial cutoff and beyond)
+    const size_t profile = sizeof(double2) * (size_t)nr;
+    const size_t row = sizeof(double) * (size_t)(16 + L.width), most = 64 << 10;
+    if (nz > 1 && 2 * profile + row <= most)
+        return sat_build<2, true>(radial, nz, nr, res, ntab, L, places, stride, sums, sat, stream);
+    if (profile + row <= most)
+        return sat_build<1, true>(radial, nz, nr, res, ntab, L, places, stride, sums, sat, stream);
+    return sat_build<1, false>(radial, nz, nr, res, ntab, L, places, stride, sums, sat, stream);
 }
 
 }  // namespace
@@ -443,17 +478,8 @@ int smx_psf_sat_build(const double* radial, int nz, int nr, double res, int peri
     if (nz == 0) return SMX_OK;
     int ntab = 2 * nr - 1;
     smx::SatLayout L = smx::make_sat_layout(ntab + 1, period);
-    if (ntab <= kSatMax) {
-        // two depths' profiles a block and the staged row while 64 KB of LDS
-        // hold them (they do up to 1 um radial cutoff and beyond)
-        const size_t profile = sizeof(double2) * (size_t)nr;
-        const size_t row = sizeof(double) * (size_t)(16 + L.width), most = 64 << 10;
-        if (nz > 1 && 2 * profile + row <= most)
-            return sat_build<2, true>(radial, nz, nr, res, ntab, L, workspace, sat, stream);
-        if (profile + row <= most)
-            return sat_build<1, true>(radial, nz, nr, res, ntab, L, workspace, sat, stream);
-        return sat_build<1, false>(radial, nz, nr, res, ntab, L, workspace, sat, stream);
-    }
+    if (ntab <= kSatMax)
+        return sat_build_any(radial, nz, nr, res, ntab, L, nullptr, L.elems(), workspace, sat, stream);
     hipLaunchKernelGGL(sat_row_kernel, dim3((ntab + 3) / 4, nz), dim3(256), 0, stream, nr, res,
                        radial, ntab, workspace);
     SMX_CHECK_LAUNCH("sat_row_kernel");
@@ -461,6 +487,37 @@ int smx_psf_sat_build(const double* radial, int nz, int nr, double res, int peri
                        workspace, L, L.elems(), sat);
     SMX_CHECK_LAUNCH("sat_col_kernel");
     return SMX_OK;
+}
+
+size_t smx_psf_sat_sorted_elems(int nr) {
+    if (nr < 2 || 2 * nr - 1 > smx::SAT_SORTED_MAX) return 0;
+    return smx::sat_sorted_elems(2 * nr);
+}
+
+int smx_sat_sorted_places(int nr, double ratio, int* places) {
+    if (nr < 2 || 2 * nr - 1 > smx::SAT_SORTED_MAX || !(ratio > 1.0) || !places) {
+        smx::set_error("smx_sat_sorted_places: invalid arguments (nr=%d, ratio=%g)", nr, ratio);
+        return SMX_EVALUE;
+    }
+    // phase of every corner; within a phase the order of the pixels
+    std::vector<std::pair<double, int>> order(2 * (size_t)nr);
+    for (int b = 0; b < 2 * nr; ++b) order[b] = {(double)b - ratio * floor((double)b / ratio), b};
+    std::stable_sort(order.begin(), order.end(),
+                     [](const auto& x, const auto& y) { return x.first < y.first; });
+    for (size_t k = 0; k < order.size(); ++k) places[order[k].second] = (int)k;
+    return SMX_OK;
+}
+
+int smx_psf_sat_build_sorted(const double* radial, int nz, int nr, double res, const int* places,
+                             double* workspace, double* sat, hipStream_t stream) {
+    if (nz < 0 || nr < 2 || 2 * nr - 1 > smx::SAT_SORTED_MAX || !radial || !places || !workspace ||
+        !sat) {
+        smx::set_error("smx_psf_sat_build_sorted: invalid arguments (nz=%d, nr=%d)", nz, nr);
+        return SMX_EVALUE;
+    }
+    if (nz == 0) return SMX_OK;
+    return sat_build_any(radial, nz, nr, res, 2 * nr - 1, smx::make_sat_layout(2 * nr, 1), places,
+                         smx::sat_sorted_elems(2 * nr), workspace, sat, stream);
 }
 
 }  // extern "C"

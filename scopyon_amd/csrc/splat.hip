@@ -14,8 +14,8 @@
 // binned to the tiles their footprint touches (count -> scan -> fill), each
 // tile's list is sorted by emitter index in LDS (so every pixel adds its
 // contributions in emitter order, like the reference loop, and the result is
-// run-to-run deterministic), then one 256-thread workgroup per tile
-// accumulates its 1024 pixels in registers.  No float atomics.
+// run-to-run deterministic), then one workgroup per tile accumulates its
+// pixels in LDS.  No float atomics in global memory.
 #include <cstdlib>
 #include <mutex>
 #include <type_traits>
@@ -38,10 +38,6 @@ using smx::WAVE_SORT_MAX;
 using smx::tile_fov_kernel;
 
 constexpr int TS = 32;         // tile side in pixels
-constexpr int TB = TS + 1;     // boundaries per tile axis
-constexpr int PY = 4;          // pixel rows per thread (256 threads x 4 = 32 x 32)
-constexpr int RS = TS / PY;    // row stride between a thread's pixels
-constexpr int CHUNK = 4;       // emitters staged in LDS per round (general path)
 constexpr int SORT_CAP = 4096; // max tile list sorted in LDS
 
 // One axis of the footprint: pixel range [k0, k1) and its cell boundaries.
@@ -128,60 +124,132 @@ __device__ inline bool emitter_tiles(const smx_fov_t& F, double xi, double yi, d
 __device__ inline int fov_of(const int* __restrict__ fov_id, int i) { return fov_id ? fov_id[i] : 0; }
 __device__ inline bool fov_ok(int f, int nfov) { return f >= 0 && f < nfov; }
 
-__global__ void bin_count_kernel(int n, const double* __restrict__ u, const double* __restrict__ v,
-                                 const double* __restrict__ w, const int* __restrict__ fov_id,
-                                 const smx_fov_t* __restrict__ fovs, int nfov, double ext_half,
-                                 int n_tiles, int* __restrict__ tile_count, int cs) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    if (!(w[i] > 0.0)) return;
-    const int f = fov_of(fov_id, i);
-    if (!fov_ok(f, nfov)) return;
-    const smx_fov_t F = fovs[f];
-    TileRange t;
-    if (!emitter_tiles(F, u[i] - F.p0u, v[i] - F.p0v, ext_half, t)) return;
-    for (int r = t.r0; r <= t.r1; ++r)
-        for (int c = t.c0; c <= t.c1; ++c)
-        {
-            int tile = F.tile_off + r * F.tiles_c + c;
-            if (tile >= 0 && tile < n_tiles) atomicAdd(&tile_count[(size_t)tile * cs], 1);
+// Tile counts and slot claims aggregate per block in LDS (BIN_THREADS
+// emitters, a window of BIN_WIN tiles from the first tile of the block's
+// first FOV): device-scope atomics are the cost of binning.
+constexpr int REC_THREADS = smx::BIN_THREADS;
+constexpr int REC_WIN = smx::BIN_WIN;
+
+__device__ inline int window_base(const int* __restrict__ fov_id, const smx_fov_t* __restrict__ fovs,
+                                  int nfov, int n) {
+    const int i0 = blockIdx.x * REC_THREADS;
+    const int f0 = i0 < n ? fov_of(fov_id, i0) : -1;
+    return fov_ok(f0, nfov) ? fovs[f0].tile_off : 0;
+}
+
+// Count the tiles of range t for the block's LDS window (or the device
+// counters outside it).
+__device__ inline void count_entries(const smx_fov_t& F, const TileRange& t, int n_tiles,
+                                     int* s_hist, int wbase, int* __restrict__ tile_count, int cs) {
+    for (int a = t.r0; a <= t.r1; ++a)
+        for (int b = t.c0; b <= t.c1; ++b) {
+            const int tile = F.tile_off + a * F.tiles_c + b;
+            if (tile >= 0 && tile < n_tiles) smx::bin_count(s_hist, wbase, tile, tile_count, cs);
         }
 }
 
-__global__ void bin_fill_kernel(int n, const double* __restrict__ u, const double* __restrict__ v,
-                                const double* __restrict__ w, const int* __restrict__ fov_id,
-                                const smx_fov_t* __restrict__ fovs, int nfov, double ext_half,
-                                int n_tiles, const int* __restrict__ tile_begin,
-                                int* __restrict__ tile_left, int cs,
-                                int* __restrict__ list, long long capacity, int* __restrict__ status) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    if (!(w[i] > 0.0)) return;
-    const int f = fov_of(fov_id, i);
-    if (!fov_ok(f, nfov)) return;
-    const smx_fov_t F = fovs[f];
+// Entries of emitter i into its tiles' lists, by the whole block (`in`: the
+// thread has an emitter with tile range t in FOV F).  Entries of a footprint
+// within 2 x 2 tiles of the window take an LDS rank, the block claims each
+// window tile's slots with one global atomic, and the entries are written at
+// claim + rank; other entries claim a slot each.
+__device__ inline void fill_entries(bool in, int i, const smx_fov_t* F, const TileRange& t,
+                                    int n_tiles, int* s_hist, int wbase,
+                                    const int* __restrict__ tile_begin,
+                                    int* __restrict__ tile_left, int cs, int* __restrict__ list,
+                                    long long capacity, int* __restrict__ status) {
+    int ent[4];   // window entries: tile offset << 16 | LDS rank (-1: none)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) ent[q] = -1;
+    if (in) {
+        const bool small = t.r1 - t.r0 <= 1 && t.c1 - t.c0 <= 1;
+        int q = 0;
+        for (int a = t.r0; a <= t.r1; ++a)
+            for (int b = t.c0; b <= t.c1; ++b) {
+                const int tile = F->tile_off + a * F->tiles_c + b;
+                if (tile < 0 || tile >= n_tiles) continue;
+                const unsigned d = (unsigned)(tile - wbase);
+                if (small && d < (unsigned)REC_WIN) {
+                    // ranks stay below 2^16: at most REC_THREADS entries per tile
+                    ent[q & 3] = (int)(d << 16) | atomicAdd(&s_hist[d], 1);
+                    ++q;
+                } else {
+                    const int pos = atomicSub(&tile_left[(size_t)tile * cs], 1) - 1;
+                    const long long at = (long long)tile_begin[tile] + pos;
+                    if (at < capacity) list[at] = i;
+                    else atomicOr(status, 2);
+                }
+            }
+    }
+    __syncthreads();
+    smx::bin_claim(s_hist, wbase, tile_left, cs);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        if (ent[q] < 0) continue;
+        const int d = ent[q] >> 16, rank = ent[q] & 0xffff;
+        const long long at = (long long)tile_begin[wbase + d] + s_hist[d] + rank;
+        if (at < capacity) list[at] = i;
+        else atomicOr(status, 2);
+    }
+}
+
+// Binning without table records (general pixel size): 100,000 emitters with
+// ~3.8 tiles each 17 us, 48 us with one device atomic per entry.
+__device__ inline bool sat_tiles(int i, int n, const double* __restrict__ u,
+                                 const double* __restrict__ v, const double* __restrict__ w,
+                                 const int* __restrict__ fov_id, const smx_fov_t* __restrict__ fovs,
+                                 int nfov, double ext_half, int& f, TileRange& t) {
+    if (i >= n || !(w[i] > 0.0)) return false;
+    f = fov_of(fov_id, i);
+    return fov_ok(f, nfov) &&
+           emitter_tiles(fovs[f], u[i] - fovs[f].p0u, v[i] - fovs[f].p0v, ext_half, t);
+}
+
+__global__ void __launch_bounds__(REC_THREADS) bin_count_kernel(
+        int n, const double* __restrict__ u, const double* __restrict__ v,
+        const double* __restrict__ w, const int* __restrict__ fov_id,
+        const smx_fov_t* __restrict__ fovs, int nfov, double ext_half, int n_tiles,
+        int* __restrict__ tile_count, int cs) {
+    __shared__ int s_hist[REC_WIN];
+    smx::bin_hist_clear(s_hist);
+    const int wbase = window_base(fov_id, fovs, nfov, n);
+    __syncthreads();
+    const int i = blockIdx.x * REC_THREADS + threadIdx.x;
+    int f = 0;
     TileRange t;
-    if (!emitter_tiles(F, u[i] - F.p0u, v[i] - F.p0v, ext_half, t)) return;
-    for (int r = t.r0; r <= t.r1; ++r)
-        for (int c = t.c0; c <= t.c1; ++c) {
-            int tile = F.tile_off + r * F.tiles_c + c;
-            if (tile < 0 || tile >= n_tiles) continue;
-            int pos = atomicSub(&tile_left[(size_t)tile * cs], 1) - 1;   // counts run down to 0
-            long long at = (long long)tile_begin[tile] + pos;
-            if (at < capacity) list[at] = i;
-            else atomicOr(status, 2);
-        }
+    if (sat_tiles(i, n, u, v, w, fov_id, fovs, nfov, ext_half, f, t))
+        count_entries(fovs[f], t, n_tiles, s_hist, wbase, tile_count, cs);
+    __syncthreads();
+    smx::bin_count_flush(s_hist, wbase, tile_count, cs);
+}
+
+__global__ void __launch_bounds__(REC_THREADS) bin_fill_kernel(
+        int n, const double* __restrict__ u, const double* __restrict__ v,
+        const double* __restrict__ w, const int* __restrict__ fov_id,
+        const smx_fov_t* __restrict__ fovs, int nfov, double ext_half, int n_tiles,
+        const int* __restrict__ tile_begin, int* __restrict__ tile_left, int cs,
+        int* __restrict__ list, long long capacity, int* __restrict__ status) {
+    __shared__ int s_hist[REC_WIN];
+    smx::bin_hist_clear(s_hist);
+    const int wbase = window_base(fov_id, fovs, nfov, n);
+    __syncthreads();
+    const int i = blockIdx.x * REC_THREADS + threadIdx.x;
+    int f = 0;
+    TileRange t = {0, 0, 0, 0};
+    const bool in = sat_tiles(i, n, u, v, w, fov_id, fovs, nfov, ext_half, f, t);
+    fill_entries(in, i, fovs + f, t, n_tiles, s_hist, wbase, tile_begin, tile_left, cs, list,
+                 capacity, status);
 }
 
 // --------------------------------------------------------------------------
-// Tile accumulation
+// Tile accumulation (general pixel size)
 // --------------------------------------------------------------------------
 struct TileArgs {
     const double* u;
     const double* v;
     const double* w;
     const int* key;          // SAT slot per emitter
-    const int* fov_id;
     const smx_fov_t* fovs;
     int nfov;
     const int* tile_fov;     // FOV of each global tile
@@ -191,7 +259,8 @@ struct TileArgs {
     const double* sat;
     size_t sat_stride;
     int n_slots;             // tables available in sat
-    smx::SatLayout L;
+    smx::SatLayout L;        // layout without `places`
+    const int* places;       // sorted layout: place of corner 0 .. ntab (NULL: L)
     double res, ext_half, unit_area;
     int ntab;
     int accumulate;          // 1: out += acc ; 0: out = acc
@@ -200,22 +269,112 @@ struct TileArgs {
     int* status;             // status word (bits as smx_splat_expected documents)
 };
 
-__global__ void __launch_bounds__(256) splat_tile_kernel(TileArgs A) {
-    // LDS: the sort buffer is only live before the main loop; the corner
-    // staging area reuses it afterwards.
+// A tile is 2 x 2 quadrants of 16 x 16 pixels; its sorted list is cut into
+// SPARTS pieces, and a wave takes one quadrant of one piece (own accumulator,
+// the pieces added at the end), so a frame of 1024 tiles runs 8192 waves.
+// Per chunk of 64 entries a wave clips the footprints to its quadrant,
+// compacts the hits, and for eight of them at a time computes the cell
+// boundaries of their edges (one lane an edge) as table places in LDS.  Then,
+// a footprint at a time in list order, its lanes take the (rows + 1) x
+// (columns + 1) corners, 64 at a time and each loaded once, into LDS while the
+// footprint before is added up from there, four corners a pixel.
+//
+// What bounds it is the traffic of the corner loads: the table of a depth key
+// is 32 MB, hardly two emitters of a frame share one, and an emitter needs 32
+// x 32 corners a pixel apart.  In the sorted layout (SatSorted) the corners of
+// one footprint row are one run of 32 doubles; the first corner of a row (cell
+// 0, always 0) and the last (cell ntab) would each be a line of their own, so
+// they are read from two vectors beside the table whose rows are runs too.
+// 100,000 emitters over 1002 keys on 1024 x 1024 pixels of 66.4 cells:
+// 1.71 ms and 7 GB with corners a tile at a time through LDS from a layout
+// with runs of 2.6 corners, 0.69 ms and 1.5 GB so (0.85 ms with four corner
+// loads per pixel instead of one per corner: the load path's address
+// processing; 0.57 ms when four tables serve every emitter, so what remains is
+// mostly instructions, VALU and LDS, not memory).  Two pieces a quadrant, 51 KB
+// of LDS and at most 80 registers: three blocks a CU; one piece 0.71 ms, four
+// 0.71-0.74 ms.
+constexpr int SPARTS = 2;
+constexpr int SQS = 16, SAS = SQS + 1;        // quadrant side, accumulator row stride
+constexpr int STHREADS = 64 * 4 * SPARTS;
+constexpr int SHITS = 8;                      // footprints with edges in LDS at a time
+constexpr int SEDGES = SQS + 1;               // edges per axis of a quadrant
+constexpr int SCORN = (SEDGES * SEDGES + 63) / 64;   // corner loads of a whole quadrant
+
+// Corner a of one axis as a table place, as byte offsets: `main` along a row's
+// run (columns) or of the row (rows); `side` of the row in the side vectors.
+// WIDE: tables of 4 GB and more, offsets in elements (never sorted).
+template <bool WIDE>
+struct SatPlaces {
+    static constexpr unsigned UNIT = WIDE ? 1 : 8;
+    const int* places;
+    smx::SatLayout L;
+    int ntab;
+    __device__ int2 row(int a) const {
+        if (WIDE || !places) {
+            const int r = (int)((unsigned)L.row_part(a) * UNIT);
+            return make_int2(r, r);
+        }
+        const int p = places[a];
+        return make_int2(p * (ntab + 1) * 8, p * 8);
+    }
+    // bit 0: the offset goes with the row's `side` instead of its `main`
+    __device__ int col(int b) const {
+        if (WIDE || !places) return (int)((unsigned)L.col_part(b) * UNIT);
+        const int side = ntab + 1;
+        if (b == 0) return (side * side * 8) | 1;
+        if (b == ntab) return ((side + 1) * side * 8) | 1;
+        return places[b] * 8;
+    }
+};
+
+// Per wave: table places of the edges of up to SHITS clipped footprints, and
+// the corners of one, row by row.
+struct SatWaveLds {
+    double corner[SCORN * 64];
+    int2 row[SHITS][SEDGES];
+    int col[SHITS][SEDGES];
+};
+
+// Corners of footprint hb + j, 64 at a time: out[q] is corner q * 64 + lane of
+// its (rows + 1) x (columns + 1), whatever the last corner holds past the end.
+template <bool WIDE>
+__device__ inline void load_corners(const TileArgs& A, const SatWaveLds& wl, int hb, int j, int rect,
+                                    int slot, int magic1, int lane, double* out) {
+    const int rc = __builtin_amdgcn_readlane(rect, hb + j);
+    const int r0 = rc & 31, c0 = rc >> 16 & 31;
+    const int W1 = (rc >> 24 & 31) - c0 + 1, n1 = W1 * ((rc >> 8 & 31) - r0 + 1);
+    const int mg = __builtin_amdgcn_readlane(magic1, hb + j);
+    const char* const T = (const char*)(
+            A.sat + (size_t)__builtin_amdgcn_readlane(slot, hb + j) * A.sat_stride);
+    const int2* const rows = wl.row[j] + r0;
+    const int* const cols = wl.col[j] + c0;
+#pragma unroll
+    for (int q = 0; q < SCORN; ++q) {
+        out[q] = 0.0;
+        if (q * 64 >= n1) continue;
+        const int idx = min(q * 64 + lane, n1 - 1);
+        const int row = (int)(__umul24((unsigned)idx, (unsigned)mg) >> 16);
+        const int2 r = rows[row];
+        const int col = cols[idx - __mul24(row, W1)];
+        if (WIDE)
+            out[q] = smx::gload((const double*)T + ((unsigned)r.x + (unsigned)col));
+        else
+            out[q] = smx::gload((const double*)(T + ((unsigned)(col & 1 ? r.y : r.x) +
+                                                     (unsigned)(col & ~1))));
+    }
+}
+
+template <bool WIDE>
+__global__ void __launch_bounds__(STHREADS, 6) splat_tile_kernel(TileArgs A) {
+    // the list is sorted in the same space first
     __shared__ union {
-        int list[SORT_CAP];
-        double corner[CHUNK][TB][TB];
-    } u;
-    __shared__ int s_id[CHUNK];
-    __shared__ int s_k0[CHUNK][2], s_k1[CHUNK][2];
-    __shared__ double s_o[CHUNK][2];
-    __shared__ int s_B[CHUNK][2][TB];          // cell boundary per tile edge (-1: outside)
-    __shared__ long long s_P[CHUNK][2][TB];    // SAT index part of that boundary
-    __shared__ double s_w[CHUNK];
-    __shared__ long long s_sat_off[CHUNK];
-    __shared__ int s_lo[CHUNK][2], s_n[CHUNK][2];   // valid tile-edge range per axis
-    __shared__ int s_off[CHUNK + 1];                 // prefix of valid corners per emitter
+        struct {
+            double acc[4 * SPARTS * SQS * SAS + 64];   // + one spill slot a lane
+            SatWaveLds wave[4 * SPARTS];
+        } t;
+        int sort[2 * SORT_CAP];
+    } lds;
+    double* const s_acc = lds.t.acc;
 
     const int tile = A.xcd ? smx::xcd_tile(blockIdx.x, gridDim.x) : (int)blockIdx.x;
     const int fov = A.tile_fov[tile];
@@ -223,8 +382,10 @@ __global__ void __launch_bounds__(256) splat_tile_kernel(TileArgs A) {
     const smx_fov_t F = A.fovs[fov];
     const int local = tile - F.tile_off;
     const int tr = local / F.tiles_c, tc = local % F.tiles_c;
-    const int ty = threadIdx.x / TS, tx = threadIdx.x % TS;   // rows ty + RS*q, column tx
-    const int pj = tc * TS + tx;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int quad = wave & 3, part = wave >> 2;
+    const int qr0 = tr * TS + (quad >> 1) * SQS, qc0 = tc * TS + (quad & 1) * SQS;
+    const int qh = min(SQS, F.nw - qr0), qw = min(SQS, F.nh - qc0);
 
     const int begin = A.tile_begin[tile];
     int count = A.tile_begin[tile + 1] - begin;
@@ -234,131 +395,140 @@ __global__ void __launch_bounds__(256) splat_tile_kernel(TileArgs A) {
     // sort the tile list by emitter index (emitter order per pixel) and write
     // it back in place
     if (count > 1 && count <= SORT_CAP) {
-        int np2 = 1;
-        while (np2 < count) np2 <<= 1;
-        for (int k = threadIdx.x; k < np2; k += blockDim.x) u.list[k] = k < count ? list[k] : 0x7fffffff;
-        __syncthreads();
-        lds_bitonic_sort(u.list, np2);
-        for (int k = threadIdx.x; k < count; k += blockDim.x) list[k] = u.list[k];
+        int* const s_sort = lds.sort;
+        if (count <= 256) smx::rank_sort(list, count, s_sort + SORT_CAP, s_sort);
+        else if (count <= 2 * STHREADS) smx::merge_rank_sort<2>(list, count, s_sort + SORT_CAP, s_sort);
+        else if (count <= 4 * STHREADS) smx::merge_rank_sort<4>(list, count, s_sort + SORT_CAP, s_sort);
+        else smx::merge_rank_sort<SORT_CAP / STHREADS>(list, count, s_sort + SORT_CAP, s_sort);
+        for (int k = threadIdx.x; k < count; k += STHREADS) list[k] = s_sort[k];
         __syncthreads();
     }
+    for (int k = threadIdx.x; k < 4 * SPARTS * SQS * SAS; k += STHREADS) s_acc[k] = 0.0;
+    __syncthreads();
 
-    double acc[PY];
-#pragma unroll
-    for (int q = 0; q < PY; ++q) acc[q] = 0.0;
-    for (int base = 0; base < count; base += CHUNK) {
-        const int nc = min(CHUNK, count - base);
-        // phase A0: per emitter and axis, the footprint range and cell origin
-        if (threadIdx.x < nc * 2) {
-            int c = threadIdx.x >> 1, ax = threadIdx.x & 1;
-            int e = list[base + c];
-            double xi = ax == 0 ? A.u[e] - F.p0u : A.v[e] - F.p0v;
-            Axis a = make_axis(ax == 0 ? F.half_w : F.half_h, xi, A.ext_half, F.pixel_length,
-                               ax == 0 ? F.nw : F.nh);
-            s_o[c][ax] = a.o;
-            s_k0[c][ax] = (int)a.k0;
-            s_k1[c][ax] = (int)a.k1;
-            long long e0 = (long long)(ax == 0 ? tr : tc) * TS;   // first edge of the tile
-            long long lo = max(a.k0 - e0, 0LL), hi = min(a.k1 - e0, (long long)TS);
-            s_lo[c][ax] = (int)lo;
-            s_n[c][ax] = hi >= lo ? (int)(hi - lo + 1) : 0;
-            if (ax == 0) {
-                s_id[c] = e;
-                int slot = A.key[e];
-                bool ok = slot >= 0 && slot < A.n_slots;
-                s_w[c] = ok ? A.w[e] : 0.0;
-                s_sat_off[c] = ok ? (long long)slot * (long long)A.sat_stride : -1;
-                if (!ok) atomicOr(A.status, 8);
-            }
+    const SatPlaces<WIDE> places{A.places, A.L, A.ntab};
+    const double inv_res = 1.0 / A.res, inv_pl = 1.0 / F.pixel_length;
+    SatWaveLds& wl = lds.t.wave[wave];
+    const int acc_off = wave * SQS * SAS, spill = 4 * SPARTS * SQS * SAS + lane;
+    const int last = (int)((long long)count * (part + 1) / SPARTS);
+    for (int base = (int)((long long)count * part / SPARTS); base < last; base += 64) {
+        // footprint of entry `lane` clipped to the quadrant: rows [r0, r1),
+        // columns [c0, c1)
+        double ou = 0.0, ov = 0.0, wgt = 0.0;
+        int slot = 0, rect = 0;
+        bool hit = false;
+        if (base + lane < last && qh > 0 && qw > 0) {
+            const int e = list[base + lane];
+            slot = A.key[e];
+            const bool ok = slot >= 0 && slot < A.n_slots;
+            if (!ok) atomicOr(A.status, 8);
+            wgt = A.w[e];
+            const double bu = F.half_w + (A.u[e] - F.p0u), bv = F.half_h + (A.v[e] - F.p0v);
+            ou = bu - A.ext_half;
+            ov = bv - A.ext_half;
+            const long long lu = smx::floor_div(ou, F.pixel_length, inv_pl);
+            const long long hu = smx::ceil_div(bu + A.ext_half, F.pixel_length, inv_pl);
+            const long long lv = smx::floor_div(ov, F.pixel_length, inv_pl);
+            const long long hv = smx::ceil_div(bv + A.ext_half, F.pixel_length, inv_pl);
+            const int r0 = (int)(max(lu, (long long)qr0) - qr0);
+            const int r1 = (int)(min(hu, (long long)(qr0 + qh)) - qr0);
+            const int c0 = (int)(max(lv, (long long)qc0) - qc0);
+            const int c1 = (int)(min(hv, (long long)(qc0 + qw)) - qc0);
+            hit = ok && r1 > r0 && c1 > c0;
+            rect = (r0 & 31) | (r1 & 31) << 8 | (c0 & 31) << 16 | (c1 & 31) << 24;
         }
-        __syncthreads();
-        // phase A1: cell boundaries of this tile's edges inside each footprint
-        for (int t = threadIdx.x; t < nc * 2 * TB; t += blockDim.x) {
-            int c = t / (2 * TB), r = t % (2 * TB);
-            int ax = r / TB, m = r % TB;
-            long long k = (long long)(ax == 0 ? tr : tc) * TS + m;
-            int b = -1;
-            long long part = 0;
-            if (k >= s_k0[c][ax] && k <= s_k1[c][ax]) {
-                Axis a;
-                a.o = s_o[c][ax];
-                a.k0 = s_k0[c][ax];
-                a.k1 = s_k1[c][ax];
-                b = axis_boundary(a, k, F.pixel_length, A.res, A.ntab);
-                part = (long long)(ax == 0 ? A.L.row_part(b) : A.L.col_part(b));
-            }
-            s_B[c][ax][m] = b;
-            s_P[c][ax][m] = part;
-        }
-        __syncthreads();
-        // phase B: gather only the valid SAT corners (compacted over the chunk),
-        // four independent loads in flight per thread
-        if (threadIdx.x == 0) {
-            int run = 0;
-            for (int c = 0; c < nc; ++c) {
-                s_off[c] = run;
-                run += s_sat_off[c] >= 0 ? s_n[c][0] * s_n[c][1] : 0;
-            }
-            s_off[nc] = run;
-        }
-        __syncthreads();
+        // compaction: hit number j to lane j, in list order
+        const unsigned long long mask = __ballot(hit);
+        const int nh = __popcll(mask);
+        if (nh == 0) continue;
         {
-            const int total = s_off[nc];
-            for (int t0 = threadIdx.x; t0 < total; t0 += 4 * 256) {
-                double vals[4];
-                int dst[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    int t = t0 + q * 256;
-                    dst[q] = -1;
-                    vals[q] = 0.0;
-                    if (t < total) {
-                        int c = 0;
-                        while (c + 1 < nc && s_off[c + 1] <= t) ++c;
-                        int r = t - s_off[c];
-                        int m = s_lo[c][0] + r / s_n[c][1];
-                        int l = s_lo[c][1] + r % s_n[c][1];
-                        vals[q] = smx::gload(A.sat + s_sat_off[c] + s_P[c][0][m] + s_P[c][1][l]);
-                        dst[q] = (c * TB + m) * TB + l;
-                    }
-                }
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    if (dst[q] >= 0) (&u.corner[0][0][0])[dst[q]] = vals[q];
-            }
+            const unsigned long long below = (1ull << lane) - 1;
+            const int to = (hit ? __popcll(mask & below) : nh + __popcll(~mask & below)) * 4;
+            auto push = [&](int v) { return __builtin_amdgcn_ds_permute(to, v); };
+            auto push_f64 = [&](double v) {
+                return __hiloint2double(push(__double2hiint(v)), push(__double2loint(v)));
+            };
+            ou = push_f64(ou);
+            ov = push_f64(ov);
+            wgt = push_f64(wgt);
+            slot = push(slot);
+            rect = push(rect);
         }
-        __syncthreads();
-        // phase C: per-pixel accumulation in emitter order
-        if (pj < F.nh) {
-            for (int c = 0; c < nc; ++c) {
-                if (s_sat_off[c] < 0) continue;
-                int c0 = s_B[c][1][tx], c1 = s_B[c][1][tx + 1];
-                if (c0 < 0 || c1 < 0 || c1 <= c0) continue;
-#pragma unroll
-                for (int q = 0; q < PY; ++q) {
-                    int r = ty + RS * q;
-                    int b0 = s_B[c][0][r], b1 = s_B[c][0][r + 1];
-                    if (b0 < 0 || b1 < 0 || b1 <= b0) continue;
-                    double sv = ((u.corner[c][r + 1][tx + 1] - u.corner[c][r][tx + 1])
-                                 - u.corner[c][r + 1][tx]) + u.corner[c][r][tx];
-                    double photons = sv * A.unit_area;
-                    if (photons > 0.0) acc[q] += photons * s_w[c];
+        const int W = max((rect >> 24 & 31) - (rect >> 16 & 31), 1);
+        // row = (idx * magic) >> 16, exact for idx < 1024 and widths up to 17
+        const int magic = (65536 + W - 1) / W, magic1 = (65536 + W) / (W + 1);
+        for (int hb = 0; hb < nh; hb += SHITS) {
+            const int nb = min(SHITS, nh - hb);
+            // table places of the quadrant edges inside each footprint
+            for (int t0 = 0; t0 < nb * 2 * SEDGES; t0 += 64) {
+                const int t = t0 + lane, j = t / (2 * SEDGES), r = t - j * (2 * SEDGES);
+                const int src = min(hb + j, 63);
+                const double o0 = __shfl(ou, src), o1 = __shfl(ov, src);
+                const int rc = __shfl(rect, src);
+                const bool is_col = r >= SEDGES;
+                const int m = is_col ? r - SEDGES : r, bits = is_col ? rc >> 16 : rc;
+                if (j < nb && m >= (bits & 31) && m <= (bits >> 8 & 31)) {
+                    // the clamps apply to a footprint's first and last edge
+                    // only: the others lie in the table
+                    const double x = (double)((is_col ? qc0 : qr0) + m) * F.pixel_length -
+                                     (is_col ? o1 : o0);
+                    const long long b64 = smx::ceil_div(x, A.res, inv_res);
+                    const int b = (int)min(max(b64, 0LL), (long long)A.ntab);
+                    if (is_col) wl.col[j][m] = places.col(b);
+                    else wl.row[j][m] = places.row(b);
                 }
             }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            // one footprint at a time, its corners loaded while the one before
+            // is added up
+            double next[SCORN];
+            load_corners<WIDE>(A, wl, hb, 0, rect, slot, magic1, lane, next);
+            for (int j = 0; j < nb; ++j) {
+                const int c = hb + j;
+                const int rc = __builtin_amdgcn_readlane(rect, c);
+                const int r0 = rc & 31, c0 = rc >> 16 & 31;
+                const int Wc = (rc >> 24 & 31) - c0, ar = Wc * ((rc >> 8 & 31) - r0);
+                const int mg = __builtin_amdgcn_readlane(magic, c);
+                const double wv = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(wgt), c),
+                                                   __builtin_amdgcn_readlane(__double2loint(wgt), c));
+#pragma unroll
+                for (int q = 0; q < SCORN; ++q) wl.corner[q * 64 + lane] = next[q];
+                if (j + 1 < nb) load_corners<WIDE>(A, wl, hb, j + 1, rect, slot, magic1, lane, next);
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int q = 0; q < SQS * SQS / 64; ++q) {
+                    if (q * 64 >= ar) break;
+                    const int idx = q * 64 + lane;
+                    const bool ok = idx < ar;
+                    const int row = (int)(__umul24((unsigned)idx, (unsigned)mg) >> 16);
+                    const double* K = wl.corner + (ok ? idx + row : 0);   // row (Wc + 1) + col
+                    const double photons =
+                            (((K[Wc + 2] - K[1]) - K[Wc + 1]) + K[0]) * A.unit_area;
+                    const int to = acc_off + (r0 * SAS + c0) + idx + __mul24(row, SAS - Wc);
+                    lds_add(s_acc + (ok ? to : spill), photons > 0.0 ? photons * wv : 0.0);
+                }
+                __builtin_amdgcn_wave_barrier();
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
-        __syncthreads();
     }
-    if (pj < F.nh) {
+    __syncthreads();
+    for (int k = threadIdx.x; k < TS * TS; k += STHREADS) {
+        const int r = k / TS, c = k % TS, pi = tr * TS + r, pj = tc * TS + c;
+        if (pi >= F.nw || pj >= F.nh) continue;
+        const int q = (r / SQS) * 2 + c / SQS, at = (r % SQS) * SAS + c % SQS;
+        double acc = 0.0;
 #pragma unroll
-        for (int q = 0; q < PY; ++q) {
-            int pi = tr * TS + ty + RS * q;
-            if (pi >= F.nw) continue;
-            size_t o = (size_t)F.pix_off + (size_t)pi * F.nh + pj;
-            if (A.accumulate) {
-                if (count > 0) A.out[o] = A.out[o] + acc[q];
-            } else {
-                A.out[o] = acc[q];
-            }
+        for (int p = 0; p < SPARTS; ++p) acc += s_acc[(p * 4 + q) * SQS * SAS + at];
+        const size_t o = (size_t)F.pix_off + (size_t)pi * F.nh + pj;
+        if (A.accumulate) {
+            if (count > 0) A.out[o] = A.out[o] + acc;
+        } else {
+            A.out[o] = acc;
         }
     }
 }
@@ -503,19 +673,6 @@ __device__ inline EmitterRec make_rec(int i, int f, const double* __restrict__ u
     return r;
 }
 
-// Tile counts and slot claims aggregate per block in LDS (BIN_THREADS
-// emitters, a window of BIN_WIN tiles from the first tile of the block's
-// first FOV): device-scope atomics are the cost of binning.
-constexpr int REC_THREADS = smx::BIN_THREADS;
-constexpr int REC_WIN = smx::BIN_WIN;
-
-__device__ inline int window_base(const int* __restrict__ fov_id, const smx_fov_t* __restrict__ fovs,
-                                  int nfov, int n) {
-    const int i0 = blockIdx.x * REC_THREADS;
-    const int f0 = i0 < n ? fov_of(fov_id, i0) : -1;
-    return fov_ok(f0, nfov) ? fovs[f0].tile_off : 0;
-}
-
 // LUT-mode geometry of the records (q = 0: phase tables of the 1 nm path).
 struct LutRec {
     int q, m, c;
@@ -593,13 +750,7 @@ __global__ void __launch_bounds__(REC_THREADS) emitter_rec_kernel(
         rec[i] = r;
         TileRange t;
         if (tile_count && r.flags != 2 && r.w > 0.0 && rec_tiles(fovs[f], r, t, lts)) {
-            const smx_fov_t& F = fovs[f];
-            for (int a = t.r0; a <= t.r1; ++a)
-                for (int b = t.c0; b <= t.c1; ++b) {
-                    const int tile = F.tile_off + a * F.tiles_c + b;
-                    if (tile >= 0 && tile < n_tiles)
-                        smx::bin_count(s_hist, wbase, tile, tile_count, cs);
-                }
+            count_entries(fovs[f], t, n_tiles, s_hist, wbase, tile_count, cs);
         }
     }
     __syncthreads();
@@ -608,9 +759,6 @@ __global__ void __launch_bounds__(REC_THREADS) emitter_rec_kernel(
 
 // Tile lists from the records (phase path): the footprint is the record's
 // pixel rectangle, already computed with the reference's float64 boundaries.
-// Entries of a footprint within 2 x 2 tiles of the window take an LDS rank,
-// the block claims each window tile's slots with one global atomic, and the
-// entries are written at claim + rank; other entries claim a slot each.
 __global__ void __launch_bounds__(REC_THREADS) bin_fill_rec_kernel(
         int n, const EmitterRec* __restrict__ rec, const int* __restrict__ fov_id,
         const smx_fov_t* __restrict__ fovs, int nfov, int n_tiles,
@@ -621,46 +769,15 @@ __global__ void __launch_bounds__(REC_THREADS) bin_fill_rec_kernel(
     const int wbase = window_base(fov_id, fovs, nfov, n);
     __syncthreads();
     const int i = blockIdx.x * REC_THREADS + threadIdx.x;
-    int ent[4];   // window entries: tile offset << 16 | LDS rank (-1: none)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) ent[q] = -1;
     const int f = i < n ? fov_of(fov_id, i) : -1;
+    bool in = false;
+    TileRange t = {0, 0, 0, 0};
     if (fov_ok(f, nfov)) {
         const EmitterRec r = rec[i];
-        const smx_fov_t& F = fovs[f];
-        TileRange t;
-        if (r.flags != 2 && r.w > 0.0 && rec_tiles(F, r, t, lts)) {
-            const bool small = t.r1 - t.r0 <= 1 && t.c1 - t.c0 <= 1;
-            int q = 0;
-            for (int a = t.r0; a <= t.r1; ++a)
-                for (int b = t.c0; b <= t.c1; ++b) {
-                    const int tile = F.tile_off + a * F.tiles_c + b;
-                    if (tile < 0 || tile >= n_tiles) continue;
-                    const unsigned d = (unsigned)(tile - wbase);
-                    if (small && d < (unsigned)REC_WIN) {
-                        // ranks stay below 2^16: at most REC_THREADS entries per tile
-                        ent[q & 3] = (int)(d << 16) | atomicAdd(&s_hist[d], 1);
-                        ++q;
-                    } else {
-                        const int pos = atomicSub(&tile_left[(size_t)tile * cs], 1) - 1;
-                        const long long at = (long long)tile_begin[tile] + pos;
-                        if (at < capacity) list[at] = i;
-                        else atomicOr(status, 2);
-                    }
-                }
-        }
+        in = r.flags != 2 && r.w > 0.0 && rec_tiles(fovs[f], r, t, lts);
     }
-    __syncthreads();
-    smx::bin_claim(s_hist, wbase, tile_left, cs);
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        if (ent[q] < 0) continue;
-        const int d = ent[q] >> 16, rank = ent[q] & 0xffff;
-        const long long at = (long long)tile_begin[wbase + d] + s_hist[d] + rank;
-        if (at < capacity) list[at] = i;
-        else atomicOr(status, 2);
-    }
+    fill_entries(in, i, fovs + max(f, 0), t, n_tiles, s_hist, wbase, tile_begin, tile_left, cs,
+                 list, capacity, status);
 }
 
 // K[slot][phi_u][phi_v][du][dv] from the SATs (same arithmetic as the tile
@@ -1320,6 +1437,17 @@ static int splat_run(int n, const double* u, const double* v, const double* w, c
                      int tile_side, const DetectArgs* det = nullptr,
                      const smx_lut_t* lut = nullptr) {
     LutRec LR{0, 0, 0, 0};
+    // format SMX_K_PLACES: no phase table, K holds the places of sorted SATs
+    const int* places = nullptr;
+    if (K && k_format == SMX_K_PLACES && !lut) {
+        places = (const int*)K;
+        K = nullptr;
+        if (det || ntab > smx::SAT_SORTED_MAX || sat_stride < smx::sat_sorted_elems(ntab + 1)) {
+            smx::set_error("smx_splat_expected: sorted tables need %zu doubles each and no "
+                           "detector epilogue", smx::sat_sorted_elems(ntab + 1));
+            return SMX_EVALUE;
+        }
+    }
     if (lut) {
         // LUT mode: float32 pixel-integral tables per depth slice, four taps
         if (!K || lut->q < 1 || lut->m != 2 * lut->c + 1 || lut->c < 1 || lut->nslices < 1) {
@@ -1366,14 +1494,12 @@ static int splat_run(int n, const double* u, const double* v, const double* w, c
     SplatWorkspace ws;
     layout_workspace(n, n_tiles, list_capacity, (char*)workspace, &ws);
     const double ext_half = (res * (double)(ntab - 1)) * 0.5;   // signal_width * 0.5
-    const int nb = (n + 255) / 256;
     const int nbr = (n + REC_THREADS - 1) / REC_THREADS;
     // lists the tile pass sorts itself; longer ones are sorted after binning
     const int long_min = !K ? SORT_CAP : (lts == 4 || (lts == 5 && q32)) ? psort_cap<1>()
                                                                          : psort_cap<2>();
-    // about two tiles per emitter at these footprints; the record path bins
-    // with per-block aggregation, the SAT path with one atomic per entry
-    const int cs = K ? smx::agg_count_stride(2LL * n, n_tiles) : smx::count_stride(2LL * n, n_tiles);
+    // about two tiles per emitter at these footprints
+    const int cs = smx::agg_count_stride(2LL * n, n_tiles);
 
     if (stages & 1) {
         // a warm workspace's counters are at zero and its tile map current;
@@ -1396,7 +1522,7 @@ static int splat_run(int n, const double* u, const double* v, const double* w, c
                                    lts, LR);
                 SMX_CHECK_LAUNCH("emitter_rec_kernel");
             } else {
-                hipLaunchKernelGGL(bin_count_kernel, dim3(nb), dim3(256), 0, stream, n, u, v, w,
+                hipLaunchKernelGGL(bin_count_kernel, dim3(nbr), dim3(REC_THREADS), 0, stream, n, u, v, w,
                                    fov_id, fovs_dev, nfov, ext_half, n_tiles, ws.tile_count, cs);
                 SMX_CHECK_LAUNCH("bin_count_kernel");
             }
@@ -1424,7 +1550,7 @@ static int splat_run(int n, const double* u, const double* v, const double* w, c
                                    ws.rec, fov_id, fovs_dev, nfov, n_tiles, ws.tile_begin,
                                    ws.tile_count, cs, ws.list, list_capacity, status_dev, lts);
             else
-                hipLaunchKernelGGL(bin_fill_kernel, dim3(nb), dim3(256), 0, stream, n, u, v, w,
+                hipLaunchKernelGGL(bin_fill_kernel, dim3(nbr), dim3(REC_THREADS), 0, stream, n, u, v, w,
                                    fov_id, fovs_dev, nfov, ext_half, n_tiles, ws.tile_begin,
                                    ws.tile_count, cs, ws.list, list_capacity, status_dev);
             SMX_CHECK_LAUNCH("bin_fill_kernel");
@@ -1490,13 +1616,17 @@ static int splat_run(int n, const double* u, const double* v, const double* w, c
         return SMX_OK;
     }
     TileArgs A;
-    A.u = u; A.v = v; A.w = w; A.key = key; A.fov_id = fov_id; A.fovs = fovs_dev; A.nfov = nfov;
+    A.u = u; A.v = v; A.w = w; A.key = key; A.fovs = fovs_dev; A.nfov = nfov;
+    A.places = places;
     A.tile_fov = ws.tile_fov; A.tile_begin = ws.tile_begin; A.list = ws.list;
     A.capacity = list_capacity;
     A.sat = sat; A.sat_stride = sat_stride; A.n_slots = n_slots; A.L = smx::make_sat_layout(ntab + 1, sat_period);
     A.res = res; A.ext_half = ext_half; A.unit_area = unit_area; A.ntab = ntab;
     A.accumulate = accumulate; A.out = out; A.status = status_dev; A.xcd = xcd_map(nfov);
-    hipLaunchKernelGGL(splat_tile_kernel, dim3(n_tiles), dim3(256), 0, stream, A);
+    if (!places && A.L.elems() >= (1ull << 29))
+        hipLaunchKernelGGL(splat_tile_kernel<true>, dim3(n_tiles), dim3(STHREADS), 0, stream, A);
+    else
+        hipLaunchKernelGGL(splat_tile_kernel<false>, dim3(n_tiles), dim3(STHREADS), 0, stream, A);
     SMX_CHECK_LAUNCH("splat_tile_kernel");
     return SMX_OK;
 }

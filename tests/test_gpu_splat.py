@@ -88,3 +88,45 @@ def test_splat_deterministic(gpu):
     a = _gpu_expected(gpu, ov, parts, 0.033)
     b = _gpu_expected(gpu, ov, parts, 0.033)
     assert numpy.array_equal(a, b)
+
+
+@pytest.mark.parametrize('mag,shape,n,spread', [(241.0, (70, 45), 300, 0.6), (60.0, (33, 64), 40, 1.3),
+                                                (150.0, (16, 200), 1500, 0.55),
+                                                (23.7, (31, 31), 1, 0.1)])
+def test_sorted_tables_equal_plain_layout(gpu, mag, shape, n, spread):
+    """Pixels that are not whole cells: the splat from sorted tables (any number
+    of entries per tile, footprints across frame and quadrant edges) gives the
+    bits of the splat from the plain layout, added to what the image holds."""
+    from scopyon_amd import _device, _epifm, _lib
+    cfg = product_config({'detector': {'image_size': list(shape)}, 'magnification': mag})
+    sim = _epifm._EPIFMSimulator(_epifm.EPIFMConfigs(cfg.default, rng=numpy.random.RandomState(0)))
+    t = sim.tables
+    assert t.places is not None
+    rng = numpy.random.RandomState(int(mag))
+    t.ensure(numpy.array([0, 3, 250, -1]))
+    half = 0.5 * numpy.array(shape) * 16e-6 / mag
+    u = _device.upload(rng.uniform(-1, 1, n) * 2 * spread * half[0], device=gpu)
+    v = _device.upload(rng.uniform(-1, 1, n) * 2 * spread * half[1], device=gpu)
+    w = _device.upload(rng.uniform(0.0, 50.0, n), device=gpu)
+    key = _device.upload(rng.randint(0, 4, n), dtype=torch.int32, device=gpu)
+    start = _device.upload(rng.uniform(0.0, 1.0, shape), device=gpu)
+    got = start.clone()
+    sim.splatter.splat(u, v, w, key, sim.fovs_dev, 1, sim.geom.n_tiles, got)
+    ref = start.clone()
+    cap = n * _epifm.tiles_per_emitter(sim.configs.pixel_length, t.ntab)
+    ws = torch.empty(_lib.lib().smx_splat_workspace_bytes(n, sim.geom.n_tiles, cap),
+                     dtype=torch.uint8, device=gpu)
+    _lib.call('smx_splat_expected', n, u.data_ptr(), v.data_ptr(), w.data_ptr(), key.data_ptr(),
+              None, sim.fovs_dev.data_ptr(), 1, sim.geom.n_tiles, t.sat.data_ptr(), t.sat_elems, 4,
+              t.ntab, t.period, 1e-9, 1e-18, cap, 1, None, 0, t.m, ref.data_ptr(), ws.data_ptr(),
+              ws.numel(), sim.splatter.status.data_ptr(), _device.stream())
+    assert int(sim.splatter.status.item()) == 0
+    assert not torch.equal(got, start)
+    assert torch.equal(got, ref)
+    with pytest.raises(ValueError):      # no detector epilogue on the general path
+        _lib.call('smx_splat_detect_ts', n, u.data_ptr(), v.data_ptr(), w.data_ptr(),
+                  key.data_ptr(), None, sim.fovs_dev.data_ptr(), 1, sim.geom.n_tiles,
+                  *t.splat_tables()[:2], 4, t.ntab, t.period, 1e-9, 1e-18, cap, 0,
+                  *t.splat_tables()[2:], t.m, None, ws.data_ptr(), ws.numel(),
+                  sim.splatter.status.data_ptr(), _device.stream(), None, None, sim.det, 0, 0, 0,
+                  None, None, got.data_ptr(), 0, 32)

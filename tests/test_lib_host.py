@@ -146,3 +146,31 @@ def test_phase_fold_matches_reflection_of_cell_ranges(ntab, period):
     assert sum(len(o) for o in orbits.values()) == period
     nc = len(orbits)
     assert lib.smx_phase_fold_elems(ntab, period) == nc * (nc + 1) // 2 * mf * mf
+
+
+@pytest.mark.parametrize('nr,ratio', [(1000, 16e-6 / 241.0 / 1e-9), (1000, 16e-6 / 60.0 / 1e-9),
+                                      (500, 1.7), (37, 5.25), (2048, 106.66666666666667)])
+def test_sorted_places_make_footprints_contiguous(nr, ratio):
+    """places is a permutation of the corners, and the corners of a footprint,
+    ceil(c + ratio k) for any c, occupy consecutive places."""
+    lib = _lib.lib()
+    side = 2 * nr
+    places = numpy.empty(side, dtype=numpy.int32)
+    assert lib.smx_sat_sorted_places(nr, ratio, places.ctypes.data) == 0
+    assert sorted(places) == list(range(side))
+    rng = numpy.random.RandomState(nr)
+    for c in rng.uniform(0.0, ratio - 1.0, 50):
+        k = numpy.arange(int(side / ratio) + 2)
+        corners = numpy.ceil(c + ratio * k).astype(int)
+        got = numpy.sort(places[corners[corners < side]])
+        # corners beyond the table's last pixel are missing from the run's end
+        assert got[-1] - got[0] <= len(got) and len(got) >= int(side / ratio)
+
+
+def test_sorted_tables_limits():
+    lib = _lib.lib()
+    assert lib.smx_psf_sat_sorted_elems(1000) == 2000 * 2002
+    assert lib.smx_psf_sat_sorted_elems(2049) == 0 and lib.smx_psf_sat_sorted_elems(1) == 0
+    places = numpy.empty(8, dtype=numpy.int32)
+    for nr, ratio in ((4, 1.0), (4, float('nan')), (1, 2.5), (5000, 2.5)):
+        assert lib.smx_sat_sorted_places(nr, ratio, places.ctypes.data) == _lib.SMX_EVALUE
