@@ -901,8 +901,8 @@ __global__ void __launch_bounds__(256) sum_f64_kernel(const double* __restrict__
 // Separable splat on the matrix cores.  Per 32 x 32 tile the image is the
 // contraction  mu_tile = A B,  A[i][e] = amp_e G(i; x_e),  B[e][j] = G(j; y_e)
 // over the tile's emitters e (zero outside each emitter's window): the tile's
-// sorted list is staged SG_STAGE emitters at a time (window origin, phases,
-// amplitude in LDS), each of the SG_WAVES waves takes every SG_WAVES-th chunk
+// sorted list is staged 256 or 512 emitters at a time (phases, amplitude and
+// window origin in LDS), each of the SG_WAVES waves takes every SG_WAVES-th chunk
 // of 16 emitters, builds its factors from the phase table and adds them into
 // its own 32 x 32 MFMA accumulator, and the waves' accumulators are summed in
 // a fixed order at the end.  Inputs are rounded to the operand type (float32,
@@ -914,15 +914,26 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int SG_WAVES = 4;
 constexpr int SG_THREADS = 64 * SG_WAVES;
-constexpr int SG_STAGE = SG_THREADS;
+// emitters staged at a time: 512, so that most tiles take one round, 256 with
+// float32 operands (whose blocks need the LDS)
+template <int DT> constexpr int sg_stage() { return DT == 0 ? SG_THREADS : 2 * SG_THREADS; }
 constexpr int SG_SORT_CAP = PSORT_CAP;   // tile lists sorted in LDS (longer: after binning)
 
-// Factor rows of a chunk emitter: [0] = 0, [1 .. W] = amp * G along the rows,
-// [W + 1 ..] = 0, then the same 18 slots along the columns; an MFMA operand
-// is row[clamp(pixel - window origin, -1, W) + 1], zero outside the window
-// with no mask.
-constexpr int SG_AXIS = 18;
-constexpr int SG_ROW = 2 * SG_AXIS;
+// A chunk's factors go to LDS as the MFMA operands themselves: per wave and
+// axis a zeroed 32 x 16 block [pixel of the tile][emitter of the chunk], into
+// which each emitter writes the 16 factors of its window (amp * G along the
+// rows, G along the columns, zeros past the window) as a column of 16 rows
+// from its window origin; a lane then reads its eight emitters of one pixel
+// with one or two 16-byte loads.  SG_PAD rows between the blocks take what a
+// window writes outside the tile (never read), so no write is tested.
+// Against factor rows in emitter order, whose operands were gathered with a
+// clamped index per pixel and emitter (16 reads and ~50 VALU per chunk and
+// lane): half the VALU instructions; 1,000,000 emitters on 2048^2 in bfloat16
+// 64 -> 57 us with the bucket sort (9 us of it the sort, 27 us the chunks, the
+// rest latency of the list, the gathers and the stores).
+constexpr int SG_PAD = 16;                             // window reach: up to 15 rows on a side
+constexpr int SG_BLOCK = TS + SG_PAD;                  // rows from one block to the next
+constexpr int SG_ROWS = SG_PAD + 2 * SG_WAVES * SG_BLOCK;
 
 struct SepArgs {
     const float* x;
@@ -933,7 +944,6 @@ struct SepArgs {
     const float2* tab;   // G block of the phase table
     float inv_depth;
     int R;
-    int W;
     const smx_fov_t* frames;
     int nframes;
     const int* tile_fov;
@@ -949,16 +959,19 @@ struct SepArgs {
     int xcd;             // 1: workgroups map to tiles by smx::xcd_tile
 };
 
+template <typename E, int STAGE>
 struct SepLds {
-    int sort[SG_SORT_CAP];                // the tile's list in index order
     union alignas(16) {
-        int raw[SG_WAVES * 256];          // sorted runs of the list (merge_rank_sort)
-        float red[16 * 64];               // the waves' accumulators, summed in turn
+        struct {
+            int raw[smx::bucket_sort_ints<SG_THREADS, 4>()];   // scratch of the sort
+            int sort[SG_SORT_CAP];        // the tile's list in index order
+        } s;
+        E op[SG_ROWS][16];                // operand blocks
+        float red[SG_WAVES - 1][16 * 64]; // the waves' accumulators of other waves' rows
     } u;
-    int2 lo[SG_STAGE];                    // window origin (frame pixels)
-    float2 ph[SG_STAGE];                  // sub-pixel phases
-    float amp[SG_STAGE];
-    float fac[SG_WAVES][16][SG_ROW];       // per wave: one chunk's factors (padded rows)
+    // phases along rows and columns, amplitude, window origin in tile pixels
+    // (rows in the low 16 bits, columns above)
+    float4 em[STAGE];
     double nll[SG_WAVES];
 };
 
@@ -969,9 +982,12 @@ template <typename T> struct Frag8 { typedef T type __attribute__((ext_vector_ty
 // and its image gradient (nll_grad) in the epilogue, from the accumulators,
 // instead of a pass over the written image.
 template <int DT, bool NLL>
-__global__ void __launch_bounds__(SG_THREADS) __attribute__((amdgpu_waves_per_eu(6, 8)))
+__global__ void __launch_bounds__(SG_THREADS) __attribute__((amdgpu_waves_per_eu(5, 8)))
 sep_gemm_kernel(SepArgs A) {
-    __shared__ SepLds L;
+    typedef typename std::conditional<DT == 0, float, typename std::conditional<DT == 1, _Float16,
+                                                                                __bf16>::type>::type E;
+    constexpr int STAGE = sg_stage<DT>(), PER = STAGE / SG_THREADS;
+    __shared__ SepLds<E, STAGE> L;
     const int tile = A.xcd ? smx::xcd_tile(blockIdx.x, gridDim.x) : (int)blockIdx.x;
     // independent loads first: frame, list bounds
     const int fr = A.tile_fov[tile];
@@ -981,10 +997,10 @@ sep_gemm_kernel(SepArgs A) {
     const smx_fov_t F = A.frames[fr];
     const int local = tile - F.tile_off;
     const int tr = local / F.tiles_c, tc = local % F.tiles_c;
-    const int tid = threadIdx.x, wave = tid >> 6, l = tid & 63;
+    const int tid = threadIdx.x, l = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int m = l & 31, half = l >> 5;
-    const int row = tr * TS + m, col = tc * TS + m;   // A row / B column of this lane
-    const int R = A.R, W = A.W;
+    const int R = A.R;
     // this wave's outputs: rows 8 wave + 4 half + i (i < 4), column m
     const int pj = tc * TS + m;
     float kk[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -1000,141 +1016,167 @@ sep_gemm_kernel(SepArgs A) {
     int* list = A.list + begin;
     const bool sorted = count <= SG_SORT_CAP;
     if (count >= 2 && sorted) {
-        // up to 1024 entries: every wave sorts a run in registers and the
-        // runs are ranked against each other; longer: bitonic sort in LDS
-        if (count <= SG_WAVES * 64) {
-            smx::merge_rank_sort<1>(list, count, L.u.raw, L.sort);
-        } else if (count <= SG_WAVES * 128) {
-            smx::merge_rank_sort<2>(list, count, L.u.raw, L.sort);
-        } else if (count <= SG_WAVES * 256) {
-            smx::merge_rank_sort<4>(list, count, L.u.raw, L.sort);
+        // up to 1024 entries through buckets; longer: bitonic sort in LDS
+        if (count <= SG_THREADS) {
+            smx::bucket_sort<SG_THREADS, 1>(list, count, L.u.s.raw, L.u.s.sort);
+        } else if (count <= 2 * SG_THREADS) {
+            smx::bucket_sort<SG_THREADS, 2>(list, count, L.u.s.raw, L.u.s.sort);
+        } else if (count <= 4 * SG_THREADS) {
+            smx::bucket_sort<SG_THREADS, 4>(list, count, L.u.s.raw, L.u.s.sort);
         } else {
             int np2 = 1;
             while (np2 < count) np2 <<= 1;
-            for (int k = tid; k < np2; k += SG_THREADS) L.sort[k] = k < count ? list[k] : 0x7fffffff;
+            for (int k = tid; k < np2; k += SG_THREADS) L.u.s.sort[k] = k < count ? list[k] : 0x7fffffff;
             __syncthreads();
-            lds_bitonic_sort(L.sort, np2);
+            lds_bitonic_sort(L.u.s.sort, np2);
         }
         // the sorted list goes back in place for the binned backward
-        for (int k = tid; k < count; k += SG_THREADS) list[k] = L.sort[k];
-    } else if (count == 1) {
-        if (tid == 0) L.sort[0] = list[0];
-        __syncthreads();
+        for (int k = tid; k < count; k += SG_THREADS) list[k] = L.u.s.sort[k];
+        __syncthreads();   // the list is complete, its space becomes the operands
+    }
+    // this thread's emitters of the next round: x, y, amplitude (packed by the
+    // count pass), loaded a round ahead of use, their list entries two rounds
+    float4 next[PER];
+    int ahead[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const int i = j * SG_THREADS + tid;
+        next[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (i < count) next[j] = A.pk[list[i]];
+        ahead[j] = STAGE + i < count ? list[STAGE + i] : 0;
     }
 
     f32x16 acc;
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
-    float (*fac)[SG_ROW] = L.fac[wave];
-    // leading zero of both axes of every row (never overwritten)
-    if (l < 32) fac[l >> 1][(l & 1) * SG_AXIS] = 0.0f;
+    const int blk = SG_PAD + 2 * wave * SG_BLOCK;   // rows, then columns
+    E (*const blkA)[16] = L.u.op + blk;
+    E (*const blkB)[16] = blkA + SG_BLOCK;
     // factor build: lane (k, ax, hb) = (l / 4, (l / 2) % 2, l % 2) writes
     // window pixels 8 hb .. 8 hb + 7 of axis ax of chunk emitter k: four
     // 16-byte table loads (value, slope pairs; zero pairs past the window)
     const int fk = l >> 2, fax = (l >> 1) & 1, fhb = l & 1;
     const float4* tab4 = reinterpret_cast<const float4*>(A.tab);
-    for (int sb = 0; sb < count; sb += SG_STAGE) {
-        const int ns = min(SG_STAGE, count - sb);
-        if (tid < ns) {
-            const int e = sorted ? L.sort[sb + tid] : list[sb + tid];
-            const float4 p = A.pk[e];   // x, y, amplitude (packed by the count pass)
-            const float xe = p.x, ye = p.y;
+    struct Chunk {
+        float4 q[4];       // table pairs
+        float f, scale;    // interpolation weight; amplitude, 1, or 0 past the chunk
+        int dst;           // first factor's place (elements of the operand blocks)
+    };
+    for (int sb = 0; sb < count; sb += STAGE) {
+        const int ns = min(STAGE, count - sb);
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int i = j * SG_THREADS + tid;
+            if (i >= ns) break;
+            const float xe = next[j].x, ye = next[j].y;
             const float fx = floorf(xe), fy = floorf(ye);
-            const bool fin = finite_coord(xe) && finite_coord(ye);
-            L.lo[tid] = fin ? make_int2((int)fx - R, (int)fy - R) : make_int2(0, 0);
-            L.ph[tid] = fin ? make_float2(xe - fx, ye - fy) : make_float2(0.0f, 0.0f);
-            L.amp[tid] = fin ? p.z : 0.0f;
+            float4 em = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (finite_coord(xe) && finite_coord(ye)) {
+                // a listed window meets the tile: the limits hold by themselves
+                const int lu = min(max((int)fx - R - tr * TS, 1 - SG_PAD), TS - 1);
+                const int lv = min(max((int)fy - R - tc * TS, 1 - SG_PAD), TS - 1);
+                em = make_float4(xe - fx, ye - fy, next[j].z,
+                                 __int_as_float((lu & 0xffff) | lv << 16));
+            }
+            L.em[i] = em;
+        }
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int i = sb + STAGE + j * SG_THREADS + tid;
+            if (i < count) next[j] = A.pk[ahead[j]];
+            ahead[j] = i + STAGE < count ? list[i + STAGE] : 0;
         }
         __syncthreads();
         const int nch = (ns + 15) >> 4;
-        // this lane's table pairs, interpolation weight and scale (amplitude,
-        // 1, or 0 past the chunk) of chunk c, loaded one chunk ahead of use
-        float4 gq[4];
-        float gf = 0.0f, gs = 0.0f;
-        auto load_g = [&](int c) {
-            const int kb = c * 16, nk = min(16, ns - kb);
-            const int k = min(fk, nk - 1);
-            const float2 ph = L.ph[kb + k];
-            float f;
-            const int slot = table_slot(fax ? ph.y : ph.x, f) + fhb * 8;
+        auto load = [&](int c, Chunk& C) {
+            const int i = c * 16 + fk;
+            const float4 em = L.em[min(i, ns - 1)];
+            const int org = __float_as_int(em.w);
+            const int slot = table_slot(fax ? em.y : em.x, C.f) + fhb * 8;
             const float4* src = tab4 + (slot >> 1);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) gq[i] = src[i];
-            gf = f;
-            gs = fk < nk ? (fax ? 1.0f : L.amp[kb + k]) : 0.0f;
+            for (int k = 0; k < 4; ++k) C.q[k] = src[k];
+            C.scale = i < ns ? (fax ? 1.0f : em.z) : 0.0f;
+            C.dst = (blk + fax * SG_BLOCK + fhb * 8 + (fax ? org >> 16 : (int)(short)org)) * 16 + fk;
         };
-        if (wave < nch) load_g(wave);
-        for (int c = wave; c < nch; c += SG_WAVES) {
-            const int kb = c * 16;
+        auto add = [&](const Chunk& C) {
             float v[8];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                v[2 * i] = fmaf(gf, gq[i].y, gq[i].x) * gs;
-                v[2 * i + 1] = fmaf(gf, gq[i].w, gq[i].z) * gs;
+                v[2 * i] = fmaf(C.f, C.q[i].y, C.q[i].x) * C.scale;
+                v[2 * i + 1] = fmaf(C.f, C.q[i].w, C.q[i].z) * C.scale;
             }
-            if (c + SG_WAVES < nch) load_g(c + SG_WAVES);
-            float* dst = &fac[fk][fax * SG_AXIS + 1 + fhb * 8];
+            // zero both blocks, then the windows
+            float4* const zero = reinterpret_cast<float4*>(blkA[0]);
+            constexpr int Z = TS * 16 * (int)sizeof(E) / 16 / 64;   // 16-byte stores a lane
+            constexpr int ZB = SG_BLOCK * 16 * (int)sizeof(E) / 16;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) dst[i] = v[i];
+            for (int i = 0; i < Z; ++i) {
+                zero[i * 64 + l] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                zero[ZB + i * 64 + l] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) (&L.u.op[0][0])[C.dst + i * 16] = (E)v[i];
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            // operands: row[clamp(offset, -1, W) + 1] (rows past the chunk are zero)
-            if (DT == 0) {
-                int2 o[8];
+            // lane (m, half): pixel m of the emitters 8 half .. 8 half + 7
+            if constexpr (DT == 0) {
+                const float4* pa = reinterpret_cast<const float4*>(&blkA[m][half * 8]);
+                const float4* pb = reinterpret_cast<const float4*>(&blkB[m][half * 8]);
+                const float4 a0 = pa[0], a1 = pa[1], b0 = pb[0], b1 = pb[1];
+                const float av[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+                const float bv[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
 #pragma unroll
-                for (int j = 0; j < 8; ++j) o[j] = L.lo[kb + 2 * j + half];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int k = 2 * j + half;
-                    const int ia = min(max(row - o[j].x, -1), W) + 1;
-                    const int ib = min(max(col - o[j].y, -1), W) + 1;
-                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fac[k][ia], fac[k][SG_AXIS + ib],
-                                                               acc, 0, 0, 0);
-                }
+                for (int j = 0; j < 8; ++j)
+                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[j], bv[j], acc, 0, 0, 0);
             } else {
-                typedef typename std::conditional<DT == 1, _Float16, __bf16>::type E;
                 typedef typename Frag8<E>::type V8;
-                V8 av, bv;
-                int2 o[8];
-#pragma unroll
-                for (int t = 0; t < 8; ++t) o[t] = L.lo[kb + half * 8 + t];
-#pragma unroll
-                for (int t = 0; t < 8; ++t) {
-                    const int k = half * 8 + t;
-                    const int ia = min(max(row - o[t].x, -1), W) + 1;
-                    const int ib = min(max(col - o[t].y, -1), W) + 1;
-                    av[t] = (E)fac[k][ia];
-                    bv[t] = (E)fac[k][SG_AXIS + ib];
-                }
+                const V8 av = *reinterpret_cast<const V8*>(&blkA[m][half * 8]);
+                const V8 bv = *reinterpret_cast<const V8*>(&blkB[m][half * 8]);
                 if constexpr (DT == 1) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bv, acc, 0, 0, 0);
                 else acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc, 0, 0, 0);
             }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        };
+        // a chunk's table loads are in flight while the chunk before is added
+        Chunk even, odd;
+        if (wave < nch) load(wave, even);
+        for (int c = wave; c < nch; c += 2 * SG_WAVES) {
+            if (c + SG_WAVES < nch) load(c + SG_WAVES, odd);
+            add(even);
+            if (c + SG_WAVES >= nch) break;
+            if (c + 2 * SG_WAVES < nch) load(c + 2 * SG_WAVES, even);
+            add(odd);
         }
         __syncthreads();
     }
-    // acc[i] holds row 8 (i / 4) + 4 half + i % 4, column m of the tile.  The
-    // waves' accumulators are added into red[] in wave order, then wave w
-    // finishes rows 8 w .. 8 w + 7.
+    // acc[i] holds row 8 (i / 4) + 4 half + i % 4, column m of the tile.  Wave w
+    // finishes rows 8 w .. 8 w + 7 (acc[4 w ..]), the waves' accumulators added in
+    // wave order: of the others' through LDS, each wave in the places left by
+    // skipping its own rows.
+    float own[4];
 #pragma unroll
-    for (int w = 0; w < SG_WAVES; ++w) {
-        if (wave == w) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i)
-                L.u.red[i * 64 + l] = w == 0 ? acc[i] : L.u.red[i * 64 + l] + acc[i];
-        }
-        __syncthreads();
+    for (int i = 0; i < 16; ++i) {
+        if (i / 4 == wave) own[i % 4] = acc[i];
+        else L.u.red[wave - (wave > i / 4)][i * 64 + l] = acc[i];
     }
+    __syncthreads();
     double part = 0.0;
     if (pj < F.nh) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int pi = tr * TS + 8 * wave + 4 * half + i;
             if (pi >= F.nw) continue;
-            const float v = L.u.red[(4 * wave + i) * 64 + l];
+            float v = 0.0f;
+#pragma unroll
+            for (int w = 0; w < SG_WAVES; ++w) {
+                const float a = w == wave ? own[i]
+                                          : L.u.red[w - (w > wave)][(4 * wave + i) * 64 + l];
+                v = w == 0 ? a : v + a;
+            }
             const size_t o = (size_t)F.pix_off + (size_t)pi * F.nh + pj;
             const float mv = A.background + v;
             if (A.mu) A.mu[o] = mv;
@@ -1397,7 +1439,7 @@ int sep_gemm_run(int n, const float* x, const float* y, const float* z, const fl
     SepArgs A;
     A.x = x; A.y = y; A.z = z; A.I = I; A.pk = ws.pk; A.tab = ws.table;
     A.inv_depth = params->inv_depth;
-    A.R = params->radius; A.W = 2 * params->radius + 1;
+    A.R = params->radius;
     A.frames = frames_dev; A.nframes = nframes;
     A.tile_fov = ws.tile_fov; A.tile_begin = ws.tile_begin; A.list = ws.list;
     A.capacity = capacity; A.background = params->background;

@@ -323,6 +323,104 @@ __device__ inline void merge_rank_sort(const int* __restrict__ list, int count, 
     __syncthreads();
 }
 
+// Smallest / largest value over the wave (every lane active), on DPP moves.
+__device__ inline int wave_min(int v) {
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x111, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x112, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x114, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x118, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xa, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xc, 0xf, false));
+    return __builtin_amdgcn_readlane(v, 63);
+}
+
+// Sort of a tile list of 1 <= count <= NT * EPT distinct entries by the
+// workgroup of NT threads, through buckets of equal index ranges between the
+// list's smallest and largest entry: count the buckets, scan the counts, place
+// the entries, then rank each within its bucket.  The indices of a tile are
+// spread over those of its frame, so a bucket holds about one entry and the
+// work per entry is a few LDS operations, where merging sorted runs takes
+// log-many compare stages (clustered indices only make a bucket's ranking
+// longer, up to a rank sort of the whole list).  lds: bucket_sort_ints<NT,
+// EPT>() ints; out[] count ints.  Float bucket numbers are monotonic in the
+// entry, so buckets are in order.
+template <int NT, int EPT> constexpr int bucket_count() { return EPT > 1 ? 2 * NT : NT; }
+template <int NT, int EPT> constexpr int bucket_sort_ints() {
+    return NT * EPT + bucket_count<NT, EPT>() + 4 + 3 * (NT / 64);
+}
+template <int NT, int EPT>
+__device__ inline void bucket_sort(const int* __restrict__ list, int count, int* lds, int* out) {
+    constexpr int NB = bucket_count<NT, EPT>(), BPT = NB / NT, NW = NT / 64;
+    int* const tmp = lds;                     // NT * EPT: entries by bucket
+    int* const start = lds + NT * EPT;        // NB + 1
+    int* const part = start + NB + 4;         // per wave: min, max, bucket total
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    int v[EPT], lo = 0x7fffffff, hi = 0;
+#pragma unroll
+    for (int r = 0; r < EPT; ++r) {
+        v[r] = r * NT + t < count ? list[r * NT + t] : -1;
+        if (v[r] >= 0) {
+            lo = min(lo, v[r]);
+            hi = max(hi, v[r]);
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < BPT; ++b) start[b * NT + t] = 0;
+    lo = wave_min(lo);
+    hi = -wave_min(-hi);
+    if (lane == 0) {
+        part[wave] = lo;
+        part[NW + wave] = hi;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        lo = min(lo, part[w]);
+        hi = max(hi, part[NW + w]);
+    }
+    const float scale = (float)NB / ((float)(hi - lo) + 1.0f);
+    int bk[EPT], at[EPT];
+#pragma unroll
+    for (int r = 0; r < EPT; ++r) {
+        bk[r] = min((int)((float)(v[r] - lo) * scale), NB - 1);
+        at[r] = v[r] >= 0 ? atomicAdd(&start[bk[r]], 1) : 0;
+    }
+    __syncthreads();
+    int n[BPT], sum = 0;
+#pragma unroll
+    for (int b = 0; b < BPT; ++b) {
+        n[b] = start[t * BPT + b];
+        sum += n[b];
+    }
+    const int incl = wave_incl_scan(sum);
+    if (lane == 63) part[2 * NW + wave] = incl;
+    __syncthreads();
+    int first = incl - sum;
+#pragma unroll
+    for (int w = 0; w < NW; ++w)
+        if (w < wave) first += part[2 * NW + w];
+#pragma unroll
+    for (int b = 0; b < BPT; ++b) {
+        start[t * BPT + b] = first;
+        first += n[b];
+    }
+    if (t == NT - 1) start[NB] = first;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < EPT; ++r)
+        if (v[r] >= 0) tmp[start[bk[r]] + at[r]] = v[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < EPT; ++r) {
+        if (v[r] < 0) continue;
+        const int b0 = start[bk[r]], b1 = start[bk[r] + 1];
+        int place = b0;
+        for (int k = b0; k < b1; ++k) place += tmp[k] < v[r];
+        out[place] = v[r];
+    }
+    __syncthreads();
+}
+
 // Rank sort of a tile list of 2 <= count distinct entries by the whole
 // workgroup: every entry's rank is the number of smaller entries (broadcast
 // LDS reads, no dependent shuffle stages), so a list of up to one entry per

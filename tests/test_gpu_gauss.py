@@ -425,3 +425,36 @@ def test_mfma_forward_merge_sorted_lists(gpu):
     assert m.check_status() == 0
     ref = G.render(shapes, x, y, numpy.zeros(n), I, numpy.zeros(n, int), **kw)[0]
     numpy.testing.assert_allclose(a.view(64, 64).cpu().numpy(), ref, rtol=2e-5)
+
+
+@pytest.mark.parametrize('count', [1, 2, 15, 16, 17, 63, 65, 255, 256, 257, 511, 512, 513, 1023,
+                                   1024, 1025, 2048, 2049])
+@pytest.mark.parametrize('spread', ['even', 'clustered'])
+def test_mfma_forward_list_lengths(gpu, count, spread):
+    """One tile's list at the edges of its sort forms, of the staging rounds
+    and of the 16-emitter chunks, with the indices spread evenly over the frame
+    or in two clusters far apart; windows reach over every side of the tile.
+    Float32 operands: each pixel sums `count` non-negative terms of relative
+    error ~4 2^-24 in some order, so (count + 4) 2^-24 bounds the sum's error;
+    the bits repeat."""
+    from scopyon_amd.gauss import GaussianModel
+    rng = numpy.random.RandomState(count)
+    far = 3 * count
+    n = count + far
+    inside = (numpy.arange(count) * n // count if spread == 'even'
+              else numpy.concatenate([numpy.arange(count - count // 2),
+                                      n - 1 - numpy.arange(count // 2)]))
+    x, y = rng.uniform(96.0, 120.0, n), rng.uniform(96.0, 120.0, n)   # elsewhere
+    x[inside], y[inside] = rng.uniform(26.0, 70.0, count), rng.uniform(26.0, 70.0, count)
+    I = rng.uniform(300.0, 900.0, n)
+    m = GaussianModel([(128, 128)], method='mfma-f32', **KW)
+    args = (_dev(x), _dev(y), None, _dev(I))
+    a = m.forward(*args).clone()
+    assert torch.equal(a, m.forward(*args))
+    assert m.check_status() == 0
+    x32, y32, I32 = (v.astype(numpy.float32).astype(float) for v in (x, y, I))
+    ref = G.render([(128, 128)], x32, y32, numpy.zeros(n), I32, numpy.zeros(n, int), **KW)[0]
+    got = m.frame(a, 0).cpu().numpy().astype(float)
+    tile = (slice(32, 64), slice(32, 64))
+    bound = (count + 8) * 2.0 ** -24 * ref.max() + 2e-7 * ref.max()
+    assert numpy.abs(got[tile] - ref[tile]).max() <= bound
