@@ -410,6 +410,11 @@ size_t smx_gauss_nll_workspace_bytes(int nframes, int max_frame_pixels);
 int smx_gauss_poisson_nll(const float* mu, const float* k, const smx_fov_t* frames_dev,
                           int nframes, int max_frame_pixels, double* loss, float* grad_mu,
                           void* workspace, size_t workspace_bytes, hipStream_t stream);
+/* out[p] = grad[p] * (float)weight[f] for every pixel p of frame f (device
+ * float64 weights): the image gradient of sum_f weight[f] loss[f] from that of
+ * the losses.  Frames and max_frame_pixels as for smx_gauss_poisson_nll. */
+int smx_gauss_scale_frames(const float* grad, const double* weight, const smx_fov_t* frames_dev,
+                           int nframes, int max_frame_pixels, float* out, hipStream_t stream);
 /* Hand-written backward of smx_gauss_forward: given grad_mu = dL/dmu, writes
  * dL/dx, dL/dy, dL/dz, dL/dI per emitter (any output may be NULL) and, when
  * gsigma (device scalar) is not NULL, dL/dsigma summed over all emitters in a

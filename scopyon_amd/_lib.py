@@ -127,6 +127,7 @@ SIGNATURES.update({
     'smx_gauss_backward_workspace_bytes': (c_size_t, [c_int]),
     'smx_gauss_nll_workspace_bytes': (c_size_t, [c_int, c_int]),
     'smx_gauss_poisson_nll': (c_int, [P, P, P, c_int, c_int, P, P, P, c_size_t, P]),
+    'smx_gauss_scale_frames': (c_int, [P, P, P, c_int, c_int, P, P]),
     'smx_gauss_backward': (c_int, [c_int, P, P, P, P, P, P, c_int, ctypes.POINTER(GaussParamsT),
                                    P, P, P, P, P, P, P, c_size_t, P]),
     'smx_gauss_backward_binned': (c_int, [c_int, P, P, P, P, P, P, c_int, c_int,

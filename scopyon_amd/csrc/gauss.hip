@@ -513,13 +513,32 @@ __global__ void __launch_bounds__(256) gauss_nll_kernel(const float* __restrict_
     if (threadIdx.x == 0) partial[(size_t)f * nblk + blockIdx.x] = s_red[0];
 }
 
-__global__ void gauss_nll_finish_kernel(const double* __restrict__ partial, int nblk, int nframes,
-                                        double* __restrict__ loss) {
-    int f = blockIdx.x * blockDim.x + threadIdx.x;
+// One wave per frame: lanes take the partial sums in a fixed stride, then a
+// fixed shuffle tree.
+__global__ void __launch_bounds__(256) gauss_nll_finish_kernel(const double* __restrict__ partial,
+                                                               int nblk, int nframes,
+                                                               double* __restrict__ loss) {
+    const int f = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (f >= nframes) return;
     double s = 0.0;
-    for (int b = 0; b < nblk; ++b) s += partial[(size_t)f * nblk + b];
-    loss[f] = s;
+    for (int b = lane; b < nblk; b += 64) s += partial[(size_t)f * nblk + b];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if (lane == 0) loss[f] = s;
+}
+
+// grad[p] * weight[frame of p] (weight rounded to float32 first): the image
+// gradient of a weighted sum of the frames' losses.
+__global__ void __launch_bounds__(256) gauss_scale_frames_kernel(
+        const float* __restrict__ grad, const double* __restrict__ weight,
+        const smx_fov_t* __restrict__ frames, int per, float* __restrict__ out) {
+    const smx_fov_t F = frames[blockIdx.y];
+    const float w = (float)weight[blockIdx.y];
+    const long long npix = (long long)F.nw * F.nh;
+    const long long start = (long long)blockIdx.x * per;
+    const long long stop = min(start + (long long)per, npix);
+    for (long long p = start + threadIdx.x; p < stop; p += blockDim.x)
+        out[(size_t)F.pix_off + (size_t)p] = grad[(size_t)F.pix_off + (size_t)p] * w;
 }
 
 struct BwdArgs {
@@ -1275,7 +1294,10 @@ bool params_ok(const smx_gauss_params_t* P) {
            P->inv_depth >= 0.0f;
 }
 
-constexpr int NLL_PER = 4096;
+// pixels per block of the separate NLL: four per thread, so that one small
+// frame still runs several blocks (61 x 83 pixels: 11 us with 4096 per block,
+// 5 us so; the serial float64 logarithms of a thread set the time)
+constexpr int NLL_PER = 1024;
 
 // backward workspace: per-emitter dL/dsigma terms and their partial sums
 // (float64), then the phase table
@@ -1516,9 +1538,22 @@ int smx_gauss_poisson_nll(const float* mu, const float* k, const smx_fov_t* fram
     hipLaunchKernelGGL(gauss_nll_kernel, dim3(nblk, nframes), dim3(256), 0, stream, mu, k,
                        frames_dev, NLL_PER, (double*)workspace, grad_mu);
     SMX_CHECK_LAUNCH("gauss_nll_kernel");
-    hipLaunchKernelGGL(gauss_nll_finish_kernel, dim3((nframes + 255) / 256), dim3(256), 0, stream,
+    hipLaunchKernelGGL(gauss_nll_finish_kernel, dim3((nframes + 3) / 4), dim3(256), 0, stream,
                        (const double*)workspace, nblk, nframes, loss);
     SMX_CHECK_LAUNCH("gauss_nll_finish_kernel");
+    return SMX_OK;
+}
+
+int smx_gauss_scale_frames(const float* grad, const double* weight, const smx_fov_t* frames_dev,
+                           int nframes, int max_frame_pixels, float* out, hipStream_t stream) {
+    if (!grad || !weight || !frames_dev || nframes <= 0 || max_frame_pixels <= 0 || !out) {
+        smx::set_error("smx_gauss_scale_frames: invalid arguments (nframes=%d)", nframes);
+        return SMX_EVALUE;
+    }
+    const int nblk = (max_frame_pixels + NLL_PER - 1) / NLL_PER;
+    hipLaunchKernelGGL(gauss_scale_frames_kernel, dim3(nblk, nframes), dim3(256), 0, stream, grad,
+                       weight, frames_dev, NLL_PER, out);
+    SMX_CHECK_LAUNCH("gauss_scale_frames_kernel");
     return SMX_OK;
 }
 

@@ -183,6 +183,16 @@ class GaussianModel:
                   _device.stream())
         return self.loss
 
+    def scale_frames(self, grad_mu, weight):
+        """grad_mu with every frame's pixels times that frame's weight (float64
+        device tensor, one per frame): dL/dmu of a weighted sum of losses."""
+        weight = weight.detach().to(torch.float64).contiguous()
+        out = torch.empty_like(grad_mu)
+        _lib.call('smx_gauss_scale_frames', grad_mu.data_ptr(), weight.data_ptr(),
+                  self.frames_dev.data_ptr(), self.nframes, self.max_frame_pixels, out.data_ptr(),
+                  _device.stream())
+        return out
+
     @staticmethod
     def _binning_key(x, y, fid, p, n, cap):
         return (x.data_ptr(), x._version, y.data_ptr(), y._version,
@@ -272,11 +282,23 @@ class _NLL(torch.autograd.Function):
     def backward(ctx, g_loss):
         (grad,) = ctx.saved_tensors
         model = ctx.model
-        # per-frame upstream weights (float64) onto that frame's pixels
-        scale = torch.repeat_interleave(
-            g_loss.to(torch.float32),
-            torch.as_tensor(numpy.diff(model.pix_offsets), device=grad.device))
-        return None, grad * scale, None
+        if (torch.is_grad_enabled() and g_loss.requires_grad) or not _has_storage(g_loss):
+            # create_graph (the product stays differentiable in g_loss) and
+            # batched gradients (vmap): plain tensor operations
+            scale = torch.repeat_interleave(
+                g_loss.to(torch.float32),
+                torch.as_tensor(numpy.diff(model.pix_offsets), device=grad.device))
+            return None, grad * scale, None
+        return None, model.scale_frames(grad, g_loss), None
+
+
+def _has_storage(t):
+    """False for the wrapper tensors of vmap and the like, which no kernel can read."""
+    try:
+        t.data_ptr()
+    except RuntimeError:
+        return False
+    return True
 
 
 def render(model, x, y, z, I, sigma=None, frame_id=None):

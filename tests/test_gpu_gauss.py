@@ -458,3 +458,41 @@ def test_mfma_forward_list_lengths(gpu, count, spread):
     tile = (slice(32, 64), slice(32, 64))
     bound = (count + 8) * 2.0 ** -24 * ref.max() + 2e-7 * ref.max()
     assert numpy.abs(got[tile] - ref[tile]).max() <= bound
+
+
+@pytest.mark.parametrize('shapes', [[(61, 83)], [(32, 32), (1, 7), (40, 33), (100, 61)]])
+def test_nll_gradient_scaling(gpu, shapes):
+    """Weighted frame losses: the image gradient is 1 - k / mu times the frame's
+    weight, bit for bit as the tensor product, through expanded, batched
+    (vmap) and differentiated (create_graph) upstream gradients."""
+    from scopyon_amd.gauss import poisson_nll
+    rng = numpy.random.RandomState(len(shapes))
+    m = _model(shapes)
+    sizes = [a * b for a, b in shapes]
+    k = _dev(rng.poisson(20.0, sum(sizes)))
+    mu = _dev(rng.uniform(1.0, 40.0, sum(sizes))).requires_grad_()
+    base = torch.empty_like(mu)
+    loss = m.nll(mu.detach(), k, base).clone()
+    md, kd = mu.detach().double(), k.double()
+    want = torch.stack([t.sum() for t in (md - kd * torch.log(md)).split(sizes)])
+    # at most ~2 * 83 + 20 additions deep in float64
+    torch.testing.assert_close(loss, want, rtol=1e-13, atol=0)
+    (g,) = torch.autograd.grad(poisson_nll(m, mu, k).sum(), mu)
+    assert torch.equal(g, base)
+    w = torch.as_tensor(rng.uniform(-2.0, 2.0, len(shapes)), device='cuda')
+    per = torch.cat([t * wf.float() for t, wf in zip(base.split(sizes), w)])
+    (g,) = torch.autograd.grad((poisson_nll(m, mu, k) * w).sum(), mu)
+    assert torch.equal(g, per)
+    wr = w.clone().requires_grad_()
+    (g,) = torch.autograd.grad((poisson_nll(m, mu, k) * wr).sum(), mu, create_graph=True)
+    assert torch.equal(g, per)
+    (gw,) = torch.autograd.grad(g.sum(), wr)
+    torch.testing.assert_close(gw.float(), torch.stack([t.sum() for t in base.split(sizes)]),
+                               rtol=1e-4, atol=1e-3)
+    (gb,) = torch.autograd.grad(poisson_nll(m, mu, k), mu, torch.eye(len(shapes), device='cuda',
+                                                                     dtype=torch.float64),
+                                is_grads_batched=True)
+    for f in range(len(shapes)):
+        a = sum(sizes[:f])
+        assert torch.equal(gb[f, a:a + sizes[f]], base[a:a + sizes[f]])
+        assert gb[f].count_nonzero() == base[a:a + sizes[f]].count_nonzero()
