@@ -757,6 +757,22 @@ __global__ void __launch_bounds__(REC_THREADS) emitter_rec_kernel(
     if (tile_count) smx::bin_count_flush(s_hist, wbase, tile_count, cs);
 }
 
+// The records alone, for the tile passes that list their emitters themselves:
+// small launches, so one wave a block spreads them over the chip.
+__global__ void __launch_bounds__(64) emitter_rec_only_kernel(
+        int n, const double* __restrict__ u, const double* __restrict__ v,
+        const double* __restrict__ w, const int* __restrict__ key, const int* __restrict__ fov_id,
+        const smx_fov_t* __restrict__ fovs, int nfov, double ext_half, double res, int ntab, int P,
+        int M, int n_slots, size_t k_stride, int folded, smx::PhaseFold PF,
+        EmitterRec* __restrict__ rec, int* __restrict__ status, LutRec LR) {
+    const int i = blockIdx.x * 64 + threadIdx.x;
+    if (i >= n) return;
+    const int f = fov_of(fov_id, i);
+    rec[i] = LR.q > 0 ? make_rec_lut(i, f, u, v, w, key, fovs, nfov, n_slots, LR, status)
+                      : make_rec(i, f, u, v, w, key, fovs, nfov, ext_half, res, ntab, P, M, n_slots,
+                                 k_stride, folded, PF, status);
+}
+
 // Tile lists from the records (phase path): the footprint is the record's
 // pixel rectangle, already computed with the reference's float64 boundaries.
 __global__ void __launch_bounds__(REC_THREADS) bin_fill_rec_kernel(
@@ -832,6 +848,8 @@ __global__ void phase_fold_kernel(const double* __restrict__ K, int nslots, int 
 }
 
 struct FastArgs {
+    int n;                   // SCAN: emitters, their FOVs (NULL: 0)
+    const int* fov_id;
     const void* Kraw;        // phase table (double or float)
     const double* u;
     const double* v;
@@ -982,10 +1000,24 @@ struct SplatLds {
     static constexpr int BYTES = DET && Q_END > SPLAT_END ? Q_END : SPLAT_END;
 };
 
-template <typename KT, int QPW, bool O32, bool DET, int TAPS, int QS>
+// SCAN: no binning ran; a tile walks all records (at most SCAN_N) in index
+// order and keeps those whose footprint meets it, in LDS: already sorted, and
+// four launches (counters, scan, fill, long-list sort) less.
+constexpr int SCAN_N = 2048;
+// Emitter-tile tests (n * n_tiles) up to which the tile passes list their
+// emitters themselves.  Binning + tile pass against listing + tile pass, us,
+// 32 px tiles: 1000 emitters on 512^2 (0.26 M tests) 30.2 / 19.4, 2000 on
+// 512^2 (0.5 M) 32.3 / 23.5, on 8 x 512^2 (4.1 M) 42.5 / 37.4, on 2048^2 (8.2 M)
+// 55.8 / 75.1.  16 px tiles, whose one wave walks the records alone: 1000 on
+// 512^2 (1 M) 31.5 / 26.2, 2000 on 512^2 (2 M) 33.2 / 37.5.
+constexpr long long SCAN_TESTS = 1ll << 22, SCAN_TESTS_16 = 1ll << 20;
+
+template <typename KT, int QPW, bool O32, bool DET, int TAPS, int QS, bool SCAN>
 __global__ void __launch_bounds__(64 * QPW * QPW) __attribute__((amdgpu_waves_per_eu(SMX_SPLAT_WPE, 8)))
 splat_phase_kernel(FastArgs A, DetectArgs D) {
     using LP = SplatLds<QPW, DET, TAPS, QS>;
+    __shared__ int s_list[SCAN ? SCAN_N : 1];
+    __shared__ int s_hits[SCAN ? 2 * LP::WPT : 1];
     constexpr int AS = LP::AS;
     // 64-pixel parts in flight per group: NSLOT table loads (one 16-byte cell
     // entry per part in LUT mode)
@@ -1008,10 +1040,12 @@ splat_phase_kernel(FastArgs A, DetectArgs D) {
     (void)ACCN;
 
     const int tile = A.xcd ? smx::xcd_tile(blockIdx.x, gridDim.x) : (int)blockIdx.x;
-    const int fov = A.tile_fov[tile];
+    // without a tile map (one FOV, SCAN): its tiles are [tile_off, tile_off + rows x columns)
+    const int fov = SCAN && !A.tile_fov ? 0 : A.tile_fov[tile];
     if (fov < 0 || fov >= A.nfov) return;
     const smx_fov_t F = A.fovs[fov];
     const int local = tile - F.tile_off;
+    if (SCAN && (local < 0 || local >= F.tiles_r * F.tiles_c)) return;
     const int tr = local / F.tiles_c, tc = local % F.tiles_c;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int qr0 = tr * TSZ + (wave / QPW) * QS, qc0 = tc * TSZ + (wave % QPW) * QS;
@@ -1023,18 +1057,53 @@ splat_phase_kernel(FastArgs A, DetectArgs D) {
     const int acc_off = wave * (ACC * 8);                          // this wave's accumulator (bytes)
     const unsigned spill = (unsigned)((WPT * ACC + lane) * 8);
 
-    const int begin = A.tile_begin[tile];
-    int count = A.tile_begin[tile + 1] - begin;
-    if ((long long)begin + count > A.capacity) count = (int)max(0LL, A.capacity - begin);
-    int* list = A.list + begin;
-    const bool sorted = count <= PSORT_CAP;
+    int count = 0;
+    int* list = nullptr;
+    if constexpr (SCAN) {
+        constexpr int LTS = TSZ == 16 ? 4 : TSZ == 32 ? 5 : 6;
+        int round = 0;
+        for (int base = 0; base < A.n; base += 64 * WPT, round ^= 1) {
+            const int i = base + (int)threadIdx.x;
+            bool hit = false;
+            if (i < A.n && (A.fov_id ? A.fov_id[i] : 0) == fov) {
+                const EmitterRec& r = A.rec[i];
+                TileRange t;
+                hit = r.flags != 2 && r.w > 0.0 && rec_tiles(F, r, t, LTS) && tr >= t.r0 &&
+                      tr <= t.r1 && tc >= t.c0 && tc <= t.c1;
+            }
+            const unsigned long long mask = __ballot(hit);
+            int before = __popcll(mask & ((1ull << lane) - 1)), total = __popcll(mask);
+            if constexpr (WPT > 1) {
+                // alternating counters: one barrier a round
+                if (lane == 0) s_hits[round * WPT + wave] = total;
+                __syncthreads();
+                total = 0;
+#pragma unroll
+                for (int w = 0; w < WPT; ++w) {
+                    if (w < wave) before += s_hits[round * WPT + w];
+                    total += s_hits[round * WPT + w];
+                }
+            }
+            if (hit) s_list[count + before] = i;
+            count += total;
+        }
+        __syncthreads();
+    } else {
+        const int begin = A.tile_begin[tile];
+        count = A.tile_begin[tile + 1] - begin;
+        if ((long long)begin + count > A.capacity) count = (int)max(0LL, A.capacity - begin);
+        list = A.list + begin;
+    }
+    const bool sorted = SCAN || count <= PSORT_CAP;
     // blocks of several waves: up to one entry per thread, rank sort by the
     // whole block (its input staged after the output); up to 4 per thread,
     // every wave sorts a run in registers and the runs are ranked against each
     // other (merge_rank_sort: measured, the rank sort is the faster of the two
     // for the ~80-entry lists of 32 px tiles, the merge for longer ones)
     constexpr int RANK_MAX = WPT > 1 ? 64 * WPT : 0;
-    if (count >= 2 && count <= RANK_MAX) {
+    if (SCAN) {
+        // listed in order
+    } else if (count >= 2 && count <= RANK_MAX) {
         smx::rank_sort(list, count, s_sort + RANK_MAX, s_sort);
     } else if (count >= 2 && count <= 2 * RANK_MAX) {
         smx::merge_rank_sort<2>(list, count, s_sort + 2 * RANK_MAX, s_sort);
@@ -1051,7 +1120,7 @@ splat_phase_kernel(FastArgs A, DetectArgs D) {
         __syncthreads();
         lds_bitonic_sort(s_sort, np2);
     }
-    if (count >= 2 && sorted) {
+    if (!SCAN && count >= 2 && sorted) {
         // sorted list back in place (read per chunk below), then the space
         // becomes the accumulators
         for (int k = threadIdx.x; k < count; k += blockDim.x) list[k] = s_sort[k];
@@ -1062,7 +1131,7 @@ splat_phase_kernel(FastArgs A, DetectArgs D) {
     for (int base = 0; base < count; base += FCHUNK) {
         const int nc = min(FCHUNK, count - base);
         if (threadIdx.x < nc) {
-            int e = smx::gload(list + base + threadIdx.x);
+            const int e = SCAN ? s_list[base + threadIdx.x] : smx::gload(list + base + threadIdx.x);
             EmitterRec r = A.rec[e];
             s_e[threadIdx.x] = e;
             s_geo[threadIdx.x] = make_int4(r.lo_u, r.lo_v, r.n_u, r.n_v);
@@ -1501,7 +1570,27 @@ static int splat_run(int n, const double* u, const double* v, const double* w, c
     // about two tiles per emitter at these footprints
     const int cs = smx::agg_count_stride(2LL * n, n_tiles);
 
-    if (stages & 1) {
+    // small launches: the tile pass lists its emitters itself (the 16 and 32
+    // pixel tiles of 16 x 16 quadrants).  The capacity must hold every entry
+    // either way, so that a list too small for the binning is still refused.
+    const long long per_axis = side > 0 ? (m + side - 2) / side + 1 : 0;
+    const bool scan = K && !q32 && lts <= 5 && n > 0 && n <= SCAN_N &&
+                      (long long)n * n_tiles <= (lts == 4 ? SCAN_TESTS_16 : SCAN_TESTS) &&
+                      list_capacity >= (long long)n * per_axis * per_axis;
+    if ((stages & 1) && scan) {
+        if (nfov > 1 && !(warm && n_tiles + 1 <= smx::SCAN_MAX)) {
+            hipLaunchKernelGGL(smx::tiles_init_kernel, dim3((n_tiles + 1 + 255) / 256), dim3(256),
+                               0, stream, nfov, fovs_dev, n_tiles, ws.tile_count, cs, ws.tile_fov,
+                               ws.long_tiles);
+            SMX_CHECK_LAUNCH("tiles_init_kernel");
+        }
+        hipLaunchKernelGGL(emitter_rec_only_kernel, dim3((n + 63) / 64), dim3(64), 0, stream, n, u,
+                           v, w, key, fov_id, fovs_dev, nfov, ext_half, res, ntab, sat_period, m,
+                           n_slots,
+                           k_format == 2 ? PF.elems() : smx_phase_table_elems(sat_period, m),
+                           k_format == 2, PF, ws.rec, status_dev, LR);
+        SMX_CHECK_LAUNCH("emitter_rec_only_kernel");
+    } else if (stages & 1) {
         // a warm workspace's counters are at zero and its tile map current;
         // the one-workgroup scan clears the long-list count itself
         if (!(warm && n_tiles + 1 <= smx::SCAN_MAX)) {
@@ -1563,9 +1652,11 @@ static int splat_run(int n, const double* u, const double* v, const double* w, c
     if (!(stages & 2)) return SMX_OK;
     if (K) {
         FastArgs B;
+        B.n = n;
+        B.fov_id = fov_id;
         B.Kraw = K;
         B.u = u; B.v = v; B.key = key; B.fovs = fovs_dev; B.nfov = nfov;
-        B.tile_fov = ws.tile_fov; B.tile_begin = ws.tile_begin; B.list = ws.list;
+        B.tile_fov = scan && nfov == 1 ? nullptr : ws.tile_fov; B.tile_begin = ws.tile_begin; B.list = ws.list;
         B.capacity = list_capacity; B.rec = ws.rec; B.K = (const double*)K; B.M = m;
         B.sat = sat; B.sat_stride = sat_stride; B.L = smx::make_sat_layout(ntab + 1, sat_period);
         B.res = res; B.ext_half = ext_half; B.unit_area = unit_area; B.ntab = ntab;
@@ -1584,17 +1675,24 @@ static int splat_run(int n, const double* u, const double* v, const double* w, c
             using KT = decltype(kt);
             constexpr bool O = decltype(o)::value, DT = decltype(dt)::value;
             constexpr int TP = decltype(taps)::value;
-            const bool wide = q32;
-            if (lts == 4)
-                hipLaunchKernelGGL((splat_phase_kernel<KT, 1, O, DT, TP, 16>), grid, dim3(64), 0, stream, B, Dv);
-            else if (lts == 5 && wide)
-                hipLaunchKernelGGL((splat_phase_kernel<KT, 1, O, DT, TP, 32>), grid, dim3(64), 0, stream, B, Dv);
-            else if (lts == 5)
-                hipLaunchKernelGGL((splat_phase_kernel<KT, 2, O, DT, TP, 16>), grid, dim3(256), 0, stream, B, Dv);
-            else if (wide)
-                hipLaunchKernelGGL((splat_phase_kernel<KT, 2, O, DT, TP, 32>), grid, dim3(256), 0, stream, B, Dv);
-            else
-                hipLaunchKernelGGL((splat_phase_kernel<KT, 4, O, DT, TP, 16>), grid, dim3(1024), 0, stream, B, Dv);
+            auto go = [&](auto qpw, auto qs, auto sc) {
+                constexpr int Q = decltype(qpw)::value, S = decltype(qs)::value;
+                constexpr bool SC = decltype(sc)::value;
+                hipLaunchKernelGGL((splat_phase_kernel<KT, Q, O, DT, TP, S, SC>), grid,
+                                   dim3(64 * Q * Q), 0, stream, B, Dv);
+            };
+            using I1 = std::integral_constant<int, 1>;
+            using I2 = std::integral_constant<int, 2>;
+            using I4 = std::integral_constant<int, 4>;
+            using S16 = std::integral_constant<int, 16>;
+            using S32 = std::integral_constant<int, 32>;
+            if (lts == 4 && scan) go(I1(), S16(), std::true_type());
+            else if (lts == 4) go(I1(), S16(), std::false_type());
+            else if (lts == 5 && q32) go(I1(), S32(), std::false_type());
+            else if (lts == 5 && scan) go(I2(), S16(), std::true_type());
+            else if (lts == 5) go(I2(), S16(), std::false_type());
+            else if (q32) go(I2(), S32(), std::false_type());
+            else go(I4(), S16(), std::false_type());
         };
         using One = std::integral_constant<int, 1>;
         using Four = std::integral_constant<int, 4>;

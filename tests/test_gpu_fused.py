@@ -126,3 +126,49 @@ def test_fused_refuses_what_it_cannot_do(gpu):
                   None, *tail)
     with pytest.raises(ValueError):       # no phase table
         _lib.call('smx_splat_detect_ts', *args, 0, None, 0, t.m, None, *tail)
+
+
+@pytest.mark.parametrize('nfov,n', [(1, 1), (1, 63), (1, 257), (1, 2048), (3, 500), (40, 30)])
+@pytest.mark.parametrize('kind', ['folded', 'float64', 'lut'])
+def test_self_listed_tiles_equal_binned(gpu, nfov, n, kind):
+    """Up to 2048 emitters the tile passes list their emitters themselves; with
+    emitters of zero weight appended past that they are binned.  Photons and
+    counts are the same bits, for interleaved FOV ids, one and several FOVs,
+    split bin / accumulate calls and a second (warm) step."""
+    from scopyon_amd import _device, _epifm, _lib
+    from scopyon_amd.batched import BatchedSimulator
+    ov = {'detector': {'image_size': [64, 64], 'exposure_time': 0.033},
+          'magnification': 100.0, 'effects': {'photo_bleaching': {'switch': False}}}
+    shapes = [(61 + f % 3, 64 - f % 5) for f in range(nfov)]
+    rng = numpy.random.RandomState(n)
+    half = 0.5 * 64 * 1.6e-7
+    total = n * nfov
+    place = rng.uniform(-1.2 * half, 1.2 * half, (2, total))
+    fov = rng.permutation(numpy.repeat(numpy.arange(nfov), n))
+    frames = []
+    for extra in (0, 2100):
+        for side in (16, 32):
+            sim = BatchedSimulator(product_config(ov), shapes, n + (extra + nfov - 1) // nfov,
+                                   dt=0.033, seed=5, tile_side=side, keep_photons=True,
+                                   psf='lut' if kind == 'lut' else 'table',
+                                   table_precision='folded' if kind == 'lut' else kind,
+                                   lut_slices=4, lut_bins=512, lut_phases=8)
+            m = sim.n
+            pos = numpy.zeros((2, m))
+            pos[:, :total] = place
+            ids = numpy.zeros(m, dtype=numpy.int32)
+            ids[:total] = fov
+            sim.fov_id.copy_(torch.as_tensor(ids))
+            sim.set_positions(numpy.zeros(m), pos[0], pos[1])
+            sim.w[total:] = 0.0
+            for step in range(2):
+                sim.splat_detect()
+                frames.append((sim.photons.clone(), sim.adc.clone()))
+            sim.photons.zero_()
+            sim.splat('smx_splat_bin')
+            sim.splat('smx_splat_accumulate')
+            frames.append((sim.photons.clone(), frames[-1][1]))
+            assert sim.status() == 0
+    assert frames[0][0].abs().sum() > 0
+    for photons, adc in frames[1:]:
+        assert torch.equal(photons, frames[0][0]) and torch.equal(adc, frames[0][1])
