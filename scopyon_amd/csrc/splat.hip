@@ -889,7 +889,15 @@ struct DetectArgs {
 };
 
 
-constexpr int FCHUNK = 64;
+// Emitters staged in LDS per round.  In tiles of several quadrants the waves
+// compact the entries that meet their quadrant (about 2 in 5 of a 32 px tile's)
+// before they clip them, from 128 staged entries: a list of 77 entries, the
+// headline batch's average, is then one round of ~31 footprints per wave
+// instead of two rounds of 64 and 13 (@C@).  One-wave tiles meet every entry,
+// and LUT footprints (56% of a tile's entries meet a quadrant) and their
+// registers leave the staging no room: 64 there.
+template <int QPW, int TAPS> constexpr bool compacts() { return QPW > 1 && TAPS == 1; }
+template <int QPW, int TAPS> constexpr int fchunk() { return compacts<QPW, TAPS>() ? 128 : 64; }
 
 // General-path pixel integral for one emitter (used for flagged emitters).
 // Inlined: a call would need the kernel argument block in private memory.
@@ -978,6 +986,8 @@ struct SplatLds {
     // most the sort capacity) fit too
     static_assert(WPT == 1 || 2 * (4 * 64 * WPT < psort_cap<QPW>() ? 4 * 64 * WPT : psort_cap<QPW>()) <= 2 * ACCN,
                   "merge sort LDS");
+    static constexpr int FCHUNK = fchunk<QPW, TAPS>();
+    static constexpr bool COMPACT = compacts<QPW, TAPS>();
     static constexpr int GEO = (ACCN * 8 + 15) & ~15;   // int4 lo_u, lo_v (frame pixels), n_u, n_v
     static constexpr int STR = GEO + FCHUNK * 16;       // int2 table strides per pixel along u, v
     static constexpr int FLAGS = STR + FCHUNK * 8;
@@ -988,7 +998,8 @@ struct SplatLds {
     static constexpr int PW = PR + WPT * PMAX * 32;     // [WPT][PMAX] weights: double, or
                                                         // float4 tap coefficients (TAPS 4)
     static constexpr int FRAC = PW + WPT * PMAX * (TAPS == 4 ? 16 : 8);   // LUT fractions
-    static constexpr int SPLAT_END = FRAC + (TAPS == 4 ? FCHUNK * 4 : 0);
+    static constexpr int IDX = FRAC + (TAPS == 4 ? FCHUNK * 4 : 0);   // byte [WPT][FCHUNK]: a quadrant's entries
+    static constexpr int SPLAT_END = IDX + (COMPACT ? WPT * FCHUNK : 0);
     // detector epilogue: rounds of RP pixels, PPT per thread (at most 4)
     static constexpr int NT = 64 * WPT;
     static constexpr int RPMAX = 4 * NT < 1024 ? 4 * NT : 1024;
@@ -1037,11 +1048,16 @@ splat_phase_kernel(FastArgs A, DetectArgs D) {
     double (*const s_pw)[PMAX] = (double (*)[PMAX])(s_lds + LP::PW);
     float4 (*const s_pc)[PMAX] = (float4 (*)[PMAX])(s_lds + LP::PW);
     unsigned* const s_frac = (unsigned*)(s_lds + LP::FRAC);
+    constexpr int FCHUNK = LP::FCHUNK;
+    unsigned char* const s_idx = (unsigned char*)s_lds + LP::IDX + (threadIdx.x >> 6) * FCHUNK;
     (void)ACCN;
 
     const int tile = A.xcd ? smx::xcd_tile(blockIdx.x, gridDim.x) : (int)blockIdx.x;
     // without a tile map (one FOV, SCAN): its tiles are [tile_off, tile_off + rows x columns)
     const int fov = SCAN && !A.tile_fov ? 0 : A.tile_fov[tile];
+    // independent of the FOV: in flight beside its loads
+    const int begin = SCAN ? 0 : A.tile_begin[tile];
+    int count = SCAN ? 0 : A.tile_begin[tile + 1] - begin;
     if (fov < 0 || fov >= A.nfov) return;
     const smx_fov_t F = A.fovs[fov];
     const int local = tile - F.tile_off;
@@ -1057,7 +1073,6 @@ splat_phase_kernel(FastArgs A, DetectArgs D) {
     const int acc_off = wave * (ACC * 8);                          // this wave's accumulator (bytes)
     const unsigned spill = (unsigned)((WPT * ACC + lane) * 8);
 
-    int count = 0;
     int* list = nullptr;
     if constexpr (SCAN) {
         constexpr int LTS = TSZ == 16 ? 4 : TSZ == 32 ? 5 : 6;
@@ -1089,19 +1104,56 @@ splat_phase_kernel(FastArgs A, DetectArgs D) {
         }
         __syncthreads();
     } else {
-        const int begin = A.tile_begin[tile];
-        count = A.tile_begin[tile + 1] - begin;
         if ((long long)begin + count > A.capacity) count = (int)max(0LL, A.capacity - begin);
         list = A.list + begin;
     }
     const bool sorted = SCAN || count <= PSORT_CAP;
+    auto stage = [&](int at, int e, const EmitterRec& r) {
+        s_e[at] = e;
+        s_geo[at] = make_int4(r.lo_u, r.lo_v, r.n_u, r.n_v);
+        s_str[at] = make_int2(r.su, r.sv);
+        s_flags[at] = r.flags;
+        s_w[at] = r.w;
+        if (TAPS == 4) s_frac[at] = r.frac;
+        s_ko[at] = r.flags == 0 ? r.table_off : 0;
+        if (r.flags & 2) atomicOr(A.status, 8);
+    };
+    // a list of one staging round: every thread loads its entry's record while
+    // the entries are ranked, and stages it at its rank -- no sorted list, and
+    // the records' latency is spent on the ranking
+    const bool ranked = LP::COMPACT && !SCAN && count <= FCHUNK;
+    if (ranked) {
+        int* const raw = (int*)(s_lds + LP::PR);   // the parts' space
+        const int t = (int)threadIdx.x;
+        const int c4 = (count + 3) & ~3;
+        if (t < c4) {
+            const int e = t < count ? smx::gload(list + t) : 0x7fffffff;
+            raw[t] = e;
+        }
+        EmitterRec r;
+        int e = 0;
+        if (t < count) {
+            e = raw[t];
+            r = A.rec[e];
+        }
+        __syncthreads();
+        if (t < count) {
+            const int4* raw4 = (const int4*)raw;
+            int rank = 0;
+            for (int q = 0; q < (c4 >> 2); ++q) {
+                const int4 o = raw4[q];
+                rank += (o.x < e) + (o.y < e) + (o.z < e) + (o.w < e);
+            }
+            stage(rank, e, r);
+        }
+    }
     // blocks of several waves: up to one entry per thread, rank sort by the
     // whole block (its input staged after the output); up to 4 per thread,
     // every wave sorts a run in registers and the runs are ranked against each
     // other (merge_rank_sort: measured, the rank sort is the faster of the two
     // for the ~80-entry lists of 32 px tiles, the merge for longer ones)
     constexpr int RANK_MAX = WPT > 1 ? 64 * WPT : 0;
-    if (SCAN) {
+    if (SCAN || ranked) {
         // listed in order
     } else if (count >= 2 && count <= RANK_MAX) {
         smx::rank_sort(list, count, s_sort + RANK_MAX, s_sort);
@@ -1120,7 +1172,7 @@ splat_phase_kernel(FastArgs A, DetectArgs D) {
         __syncthreads();
         lds_bitonic_sort(s_sort, np2);
     }
-    if (!SCAN && count >= 2 && sorted) {
+    if (!SCAN && !ranked && count >= 2 && sorted) {
         // sorted list back in place (read per chunk below), then the space
         // becomes the accumulators
         for (int k = threadIdx.x; k < count; k += blockDim.x) list[k] = s_sort[k];
@@ -1130,41 +1182,55 @@ splat_phase_kernel(FastArgs A, DetectArgs D) {
 
     for (int base = 0; base < count; base += FCHUNK) {
         const int nc = min(FCHUNK, count - base);
-        if (threadIdx.x < nc) {
+        if (!ranked && threadIdx.x < nc) {
             const int e = SCAN ? s_list[base + threadIdx.x] : smx::gload(list + base + threadIdx.x);
-            EmitterRec r = A.rec[e];
-            s_e[threadIdx.x] = e;
-            s_geo[threadIdx.x] = make_int4(r.lo_u, r.lo_v, r.n_u, r.n_v);
-            s_str[threadIdx.x] = make_int2(r.su, r.sv);
-            s_flags[threadIdx.x] = r.flags;
-            s_w[threadIdx.x] = r.w;
-            if (TAPS == 4) s_frac[threadIdx.x] = r.frac;
-            s_ko[threadIdx.x] = r.flags == 0 ? r.table_off : 0;
-            if (r.flags & 2) atomicOr(A.status, 8);
+            stage(threadIdx.x, e, A.rec[e]);
         }
         __syncthreads();
         if (active) {
-            // footprint rectangle of chunk emitter `lane` inside this quadrant:
+            // entries whose footprint meets this quadrant, compacted in order
+            int nh = nc;
+            if constexpr (LP::COMPACT) {
+                nh = 0;
+#pragma unroll
+                for (int g0 = 0; g0 < FCHUNK; g0 += 64) {
+                    if (g0 >= nc) break;
+                    const int4 g = s_geo[g0 + lane];
+                    const bool hit = g0 + lane < nc && s_flags[g0 + lane] != 2 &&
+                                     g.x < qr0 + qh && g.x + g.z > qr0 && g.y < qc0 + qw &&
+                                     g.y + g.w > qc0;
+                    const unsigned long long mask = __ballot(hit);
+                    if (hit) s_idx[nh + __popcll(mask & ((1ull << lane) - 1))] = (unsigned char)(g0 + lane);
+                    nh += __popcll(mask);
+                }
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            }
+            for (int hb = 0; hb < (LP::COMPACT ? nh : 1); hb += 64) {
+            // footprint rectangle of this lane's entry `ix` inside the quadrant:
             // origin (rr0, cc0) in the quadrant, width W, `area` pixels in np
             // parts, kq = table element of its first pixel
+            const bool mine = hb + lane < nh;
+            const int ix = LP::COMPACT ? (int)s_idx[min(hb + lane, nh - 1)] : lane;
             int np = 0, W = 1, area = 0, rr0 = 0, cc0 = 0, su = 0, sv = 0;
             long long kq = 0;
             bool irr = false;
-            if (lane < nc && s_flags[lane] != 2) {
-                const int4 g = s_geo[lane];
+            if (mine && s_flags[ix] != 2) {
+                const int4 g = s_geo[ix];
                 const int r0 = max(g.x, qr0), r1 = min(g.x + g.z, qr0 + qh);
                 const int c0 = max(g.y, qc0), c1 = min(g.y + g.w, qc0 + qw);
                 if (r1 > r0 && c1 > c0) {
-                    const int2 st = s_str[lane];
+                    const int2 st = s_str[ix];
                     W = c1 - c0;
                     area = (r1 - r0) * W;
                     np = (area + 63) >> 6;
-                    irr = s_flags[lane] == 1;
+                    irr = s_flags[ix] == 1;
                     rr0 = r0 - qr0;
                     cc0 = c0 - qc0;
                     su = st.x;
                     sv = st.y;
-                    kq = s_ko[lane] + (long long)(r0 - g.x) * su + (long long)(c0 - g.y) * sv;
+                    kq = s_ko[ix] + (long long)(r0 - g.x) * su + (long long)(c0 - g.y) * sv;
                 }
             }
             const bool any_irregular = __ballot(irr) != 0;
@@ -1182,16 +1248,17 @@ splat_phase_kernel(FastArgs A, DetectArgs D) {
                     const int rc = __shfl(rr0, c), cc = __shfl(cc0, c);
                     const int suc = __shfl(su, c), svc = __shfl(sv, c);
                     const long long kqc = __shfl(kq, c);
+                    const int xc = __shfl(ix, c);
                     const int idx = p * 64 + lane;
                     if (idx >= ar) continue;
                     const int row = idx / Wc, col = idx - row * Wc;
                     double val;
-                    if (s_flags[c] == 1) {
-                        val = sat_pixel(A, F, s_e[c], s_w[c], qr0 + rc + row, qc0 + cc + col, 0.0);
+                    if (s_flags[xc] == 1) {
+                        val = sat_pixel(A, F, s_e[xc], s_w[xc], qr0 + rc + row, qc0 + cc + col, 0.0);
                     } else {
                         val = (double)smx::gload((const KT*)A.Kraw + kqc + (long long)row * suc +
                                                  (long long)col * svc) *
-                              s_w[c];
+                              s_w[xc];
                     }
                     lds_add(acc + (rc + row) * AS + cc + col, val);
                 }
@@ -1204,11 +1271,11 @@ splat_phase_kernel(FastArgs A, DetectArgs D) {
                 float* pwf = reinterpret_cast<float*>(pw);
                 float4* pc = s_pc[wave];
                 const int magic = (65536 + W - 1) / W;
-                const double w = lane < nc ? s_w[lane] : 0.0;
+                const double w = mine ? s_w[ix] : 0.0;
                 // LUT mode: bilinear weights of the four phase taps, times w
                 float4 cw = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (TAPS == 4 && lane < nc) {
-                    const unsigned fr = s_frac[lane];
+                if (TAPS == 4 && mine) {
+                    const unsigned fr = s_frac[ix];
                     const float fu = (float)(fr & 0xffffu) * (1.0f / 65535.0f);
                     const float fv = (float)(fr >> 16) * (1.0f / 65535.0f);
                     const float wf = (float)w;
@@ -1306,6 +1373,7 @@ splat_phase_kernel(FastArgs A, DetectArgs D) {
                     __builtin_amdgcn_wave_barrier();
                     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
                 }
+            }
             }
         }
         __syncthreads();
