@@ -23,9 +23,18 @@ def ptr(t):
     return None if t is None else t.data_ptr()
 
 
+UPLOAD_STAGED = 1 << 18   # bytes
+
+
 def upload(a, dtype=torch.float64, device=None):
     device = device or require_gpu()
     a = numpy.ascontiguousarray(a)
+    if 0 < a.nbytes <= UPLOAD_STAGED:
+        # through pinned memory: a copy from pageable memory would wait for the
+        # kernels before it on the stream (torch keeps the block until it is read)
+        src = torch.from_numpy(a)
+        staged = torch.empty(src.shape, dtype=dtype, pin_memory=True)
+        return staged.copy_(src).to(device=device, non_blocking=True)
     return torch.from_numpy(a).to(device=device, dtype=dtype, non_blocking=False)
 
 

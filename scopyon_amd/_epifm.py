@@ -305,6 +305,13 @@ def _status_check(status):
         raise ValueError('probabilities contain NaN')
 
 
+def _molecule_ids(column):
+    """[int(m) for m in column] (NaN and infinities raise as int() does)."""
+    if (numpy.abs(column) < 2.0 ** 63).all():
+        return column.astype(numpy.int64).tolist()
+    return [int(m) for m in column]
+
+
 class _EPIFMSimulator:
     """GPU counterpart of src/scopyon/_epifm.py:998-1491 (processes == 1)."""
 
@@ -328,11 +335,16 @@ class _EPIFMSimulator:
         # photobleaching: molecule id -> budget slot (device budgets)
         self._budget_slot = {}
         self._budget = torch.zeros(0, dtype=torch.float64, device=self.device)
+        self._slot_ids = self._slots = None     # the last time point's ids and their slots
         self._philox_frame = 0
 
     # ---- bleaching state (host dict <-> device array) ----
     def _bleach_slots(self, m_ids, states, rng):
         """Slots for m_ids; draws first-sight budgets in particle order (_epifm.py:1296-1301)."""
+        if m_ids == self._slot_ids:
+            return self._slots      # the molecules of the time point before
+        if len(set(m_ids)) != len(m_ids):
+            raise NotImplementedError('duplicate molecule ids within one time point')
         new = []
         slots = numpy.empty(len(m_ids), dtype=numpy.int32)
         for i, m in enumerate(m_ids):
@@ -350,26 +362,26 @@ class _EPIFMSimulator:
             vals = numpy.empty(len(new))
             amp0, _ = self.configs.snells_law()
             N_emit0 = self.configs.emit_photons(amp0, 1.0)
-            half_life = self.configs.photobleaching_half_life
-            for j, (s, m) in enumerate(new):
-                if m in states:
-                    vals[j] = states[m]
-                elif isinstance(rng, PhiloxRNG):
-                    vals[j] = rng.host_exponential(half_life / numpy.log(2.0)) * N_emit0
-                else:
-                    beta = half_life / numpy.log(2.0)
-                    vals[j] = rng.exponential(scale=beta, size=None) * N_emit0
+            beta = self.configs.photobleaching_half_life / numpy.log(2.0)
+            drawn = numpy.array([m not in states for _, m in new])
+            vals[~drawn] = [states[m] for _, m in new if m in states]
+            count = int(drawn.sum())
+            if count:      # one vector draw gives the values of as many single ones
+                vals[drawn] = (rng.host_exponentials(beta, count) if isinstance(rng, PhiloxRNG)
+                               else rng.exponential(scale=beta, size=count)) * N_emit0
             idx = _device.upload(numpy.array([s for s, _ in new]), dtype=torch.int64,
                                  device=self.device)
             self._budget[idx] = _device.upload(vals, device=self.device)
-        return _device.upload(slots, dtype=torch.int32, device=self.device)
+        self._slots = _device.upload(slots, dtype=torch.int32, device=self.device)
+        self._slot_ids = m_ids
+        return self._slots
 
     def _states_dict(self):
-        vals = self._budget.cpu().numpy()
-        return {m: float(vals[s]) if vals[s] != 0 else 0 for m, s in self._budget_slot.items()}
+        # slots are numbered in the order of the ids
+        return {m: v or 0 for m, v in zip(self._budget_slot, self._budget.tolist())}
 
     # ---- one sub-step ----
-    def _substep(self, particles, unit_time, camera, states, rng, optinfo, full_output):
+    def _substep(self, particles, unit_time, camera, states, rng, pending, full_output):
         n = len(particles)
         if n == 0:
             return
@@ -384,29 +396,27 @@ class _EPIFMSimulator:
         p_state = dev[:, 4].contiguous()
         budget = slots = None
         if states is not None and c.photobleaching_switch:
-            m_ids = [int(m) for m in p[:, 3]]
-            if len(set(m_ids)) != len(m_ids):
-                raise NotImplementedError('duplicate molecule ids within one time point')
-            slots = self._bleach_slots(m_ids, states, rng)
+            slots = self._bleach_slots(_molecule_ids(p[:, 3]), states, rng)
             budget = self._budget
         w, key, ps = self.splatter.weights(depth, p_state, unit_time, budget, slots,
                                            self.tables.slot_map())
         self.splatter.splat(u, v, w, key, self.fovs_dev, 1, self.geom.n_tiles, camera)
         if full_output:
-            self._true_data(p, unit_time, w, ps, optinfo)
+            pending.append((p, unit_time, w, ps))
 
     def _true_data(self, p, unit_time, w, ps, optinfo):
         """Per-molecule sums of _epifm.py:1321-1333."""
         w = w.cpu().numpy()
         ps = ps.cpu().numpy()
         depth = p[:, 0] - self.configs.detector_focal_point[0]
-        for i in range(len(p)):
-            m = int(p[i, 3])
-            if m not in optinfo:
-                optinfo[m] = numpy.zeros(8, dtype=numpy.float64)
-            optinfo[m] += numpy.array([
-                unit_time, unit_time * ps[i], unit_time * p[i, 1], unit_time * p[i, 2],
-                unit_time * p[i, 1], unit_time * p[i, 2], unit_time * depth[i], w[i]])
+        u, v = unit_time * p[:, 1], unit_time * p[:, 2]
+        rows = 0.0 + numpy.column_stack([numpy.full(len(p), unit_time), unit_time * ps, u, v, u, v,
+                                         unit_time * depth, w])
+        for m, row in zip(_molecule_ids(p[:, 3]), rows):
+            if m in optinfo:
+                optinfo[m] += row
+            else:
+                optinfo[m] = row.copy()
 
     # ---- detector ----
     def detector(self, camera, rng, full_output):
@@ -436,15 +446,16 @@ class _EPIFMSimulator:
         sws = _device.ARENA.get('det_scan', lib.smx_scan_workspace_bytes(n), self.device)
         _lib.call('smx_exclusive_scan_i32', n, flag.data_ptr(), uidx.data_ptr(), sws.data_ptr(),
                   sws.numel(), st)
-        count = int(uidx[-1].item()) + int(flag[-1].item())
         shape = c.detector_image_size
         # reference order: readout noise (one vector draw), then one uniform
-        # per E > 0 pixel inside RandomState.choice (_epifm.py:1449-1454, 393-400)
-        if c.detector_readout_noise <= 0:
-            noise = None
-        else:
-            noise = _device.upload(rng.normal(0, c.detector_readout_noise, shape),
-                                   device=self.device)
+        # per E > 0 pixel inside RandomState.choice (_epifm.py:1449-1454, 393-400);
+        # the noise is drawn while the GPU still forms the image
+        noise = (rng.normal(0, c.detector_readout_noise, shape) if c.detector_readout_noise > 0
+                 else None)
+        count = int((uidx[-1] + flag[-1]).item())
+        _status_check(self.splatter.status)
+        if noise is not None:
+            noise = _device.upload(noise, device=self.device)
         uni = _device.upload(rng.random_sample(count) if count else numpy.zeros(1),
                              device=self.device)
         E_common = float(c.detector_qeff * ((0.0 + c.background_mean) if c.background_switch
@@ -511,6 +522,21 @@ class _EPIFMSimulator:
     def output_frame(self, input_data, frame_index=0, start_time=0.0, exposure_time=None,
                      fluorescence_states=None, rng=None, processes=None, full_output=True):
         """_epifm.py:1121-1225."""
+        E, adc, info = self.expose(input_data, frame_index, start_time, exposure_time,
+                                   fluorescence_states, rng, full_output)
+        nw, nh = self.configs.detector_image_size
+        cam = numpy.empty((nw, nh, 2))
+        cam[:, :, 0] = self.image(E)
+        cam[:, :, 1] = self.image(adc)
+        return cam, info
+
+    def image(self, pixels):
+        """A device frame on the host, (nw, nh)."""
+        return pixels.cpu().numpy().reshape(self.configs.detector_image_size)
+
+    def expose(self, input_data, frame_index=0, start_time=0.0, exposure_time=None,
+               fluorescence_states=None, rng=None, full_output=True):
+        """One frame left on the device: (expectation, ADC counts, info)."""
         c = self.configs
         exposure_time = exposure_time or c.detector_exposure_time
         if rng is None:
@@ -530,16 +556,22 @@ class _EPIFMSimulator:
         nw, nh = c.detector_image_size
         camera = torch.zeros(nw * nh, dtype=torch.float64, device=self.device)
         self.splatter.status.zero_()
-        optinfo = {}
+        pending = []
         for i, (i_time, particles) in enumerate(frame_data):
             current = i_time if i != 0 else t
             nxt = frame_data[i + 1][0] if i + 1 < len(frame_data) else t + exposure_time
             unit_time = nxt - current
             if unit_time < 1e-13:
                 continue
-            self._substep(particles, unit_time, camera, fluorescence_states, rng, optinfo,
+            self._substep(particles, unit_time, camera, fluorescence_states, rng, pending,
                           full_output)
+        E, adc = self.detector(camera, rng, full_output)
         _status_check(self.splatter.status)
+        # the weights come to the host only now: the detector's random numbers
+        # are drawn while the GPU still forms the image
+        optinfo = {}
+        for step in pending:
+            self._true_data(*step, optinfo)
         if full_output:
             p0 = c.detector_focal_point
             pl = c.pixel_length
@@ -548,25 +580,31 @@ class _EPIFMSimulator:
                 optinfo[m_id][2:6] /= optinfo[m_id][0]
                 optinfo[m_id][2] = (optinfo[m_id][2] - p0[1]) / pl + (nw - 1) * 0.5
                 optinfo[m_id][3] = (optinfo[m_id][3] - p0[2]) / pl + (nh - 1) * 0.5
-        E, adc = self.detector(camera, rng, full_output)
-        _status_check(self.splatter.status)
-        cam = numpy.empty((nw, nh, 2))
-        cam[:, :, 0] = E.cpu().numpy().reshape(nw, nh)
-        cam[:, :, 1] = adc.cpu().numpy().reshape(nw, nh)
         info = dict(true_data=optinfo)
         if fluorescence_states is not None:
             fluorescence_states.update(self._states_dict())
             info['fluorescence_states'] = copy.copy(fluorescence_states)
-        return cam, info
+        return E, adc, info
 
     def generate_frames(self, input_data, num_frames, start_time=0.0, exposure_time=None,
                         rng=None, processes=None, full_output=True):
         """_epifm.py:1017-1049."""
+        for frame in self._frames(self.output_frame, input_data, num_frames, start_time,
+                                  exposure_time, rng, processes=processes,
+                                  full_output=full_output):
+            yield frame
+
+    def exposures(self, input_data, num_frames, start_time=0.0, exposure_time=None, rng=None,
+                  full_output=True):
+        """generate_frames with the frames left on the device (expose)."""
+        return self._frames(self.expose, input_data, num_frames, start_time, exposure_time, rng,
+                            full_output=full_output)
+
+    def _frames(self, one, input_data, num_frames, start_time, exposure_time, rng, **kwargs):
         if rng is None:
             rng = numpy.random.RandomState()
         states = {} if self.configs.photobleaching_switch else None
         exposure_time = exposure_time or self.configs.detector_exposure_time
         for k in range(num_frames):
-            yield self.output_frame(input_data, frame_index=k, start_time=start_time,
-                                    exposure_time=exposure_time, fluorescence_states=states,
-                                    rng=rng, processes=processes, full_output=full_output)
+            yield one(input_data, frame_index=k, start_time=start_time,
+                      exposure_time=exposure_time, fluorescence_states=states, rng=rng, **kwargs)

@@ -95,12 +95,11 @@ class EPIFMSimulator(object):
         """One frame; returns Image (and the info dict when full_output)."""
         data = self.__format_inputs(inputs)
         base = self.base()
-        camera, infodict = base.output_frame(data, start_time=start_time,
-                                             exposure_time=exposure_time, rng=self.__rng,
-                                             full_output=full_output)
-        img = _image.Image(camera[:, :, 1])
+        E, adc, infodict = base.expose(data, start_time=start_time, exposure_time=exposure_time,
+                                       rng=self.__rng, full_output=full_output)
+        img = _image.Image(base.image(adc))
         if full_output:
-            infodict.update(dict(expectation=camera[:, :, 0]))
+            infodict.update(dict(expectation=base.image(E)))
             return img, infodict
         return img
 
@@ -109,12 +108,12 @@ class EPIFMSimulator(object):
         """A generator of frames; photobleaching state persists across them."""
         data = self.__format_inputs(inputs)
         base = self.base()
-        for camera, infodict in base.generate_frames(data, num_frames, start_time=start_time,
-                                                     exposure_time=exposure_time, rng=self.__rng,
-                                                     full_output=full_output):
-            img = _image.Image(camera[:, :, 1])
+        for E, adc, infodict in base.exposures(data, num_frames, start_time=start_time,
+                                               exposure_time=exposure_time, rng=self.__rng,
+                                               full_output=full_output):
+            img = _image.Image(base.image(adc))
             if full_output:
-                infodict.update(dict(expectation=camera[:, :, 0]))
+                infodict.update(dict(expectation=base.image(E)))
                 yield img, infodict
             else:
                 yield img

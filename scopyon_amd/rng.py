@@ -26,5 +26,9 @@ class PhiloxRNG:
     def host_exponential(self, scale):
         return float(self._host.exponential(scale))
 
+    def host_exponentials(self, scale, n):
+        """n draws of host_exponential(scale), in order."""
+        return self._host.exponential(scale, n)
+
     def __repr__(self):
         return 'PhiloxRNG(seed={})'.format(self.seed)

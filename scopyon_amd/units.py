@@ -7,6 +7,7 @@ same behaviour for the units scopyon configurations use: ``to_base_units()``
 to SI magnitudes, dimensionality checks raising ``DimensionalityError`` and the
 ``'{:~}'`` short format.
 """
+import functools
 import math
 import numbers
 import re
@@ -102,7 +103,14 @@ def parse_units(text):
     """'kg / s ** 3' -> (factor to SI, {dim: power})."""
     if text is None:
         return 1.0, {}
-    toks = _tokens(str(text))
+    f, d = _parse(str(text))
+    return f, dict(d)
+
+
+# a simulator reads some forty leaves of a few distinct units per frame
+@functools.lru_cache(maxsize=256)
+def _parse(text):
+    toks = _tokens(text)
     pos = [0]
 
     def peek():

@@ -74,6 +74,36 @@ def test_generate_images_bleaching_matches_oracle(gpu):
             assert st[m] == pytest.approx(ost[m], rel=1e-12, abs=0)
 
 
+def test_bleaching_with_molecules_coming_and_going(gpu):
+    """Molecule sets that stay, shrink, come back in another order and grow over
+    the sub-steps: budgets are drawn in order of first sight and follow the ids."""
+    import scopyon_amd
+    ov = {'detector': {'image_size': [24, 24], 'exposure_time': 0.033}, 'magnification': 100.0,
+          'effects': {'photo_bleaching': {'switch': True, 'half_life': 0.03}}}
+    pl = 16e-6 / 100.0
+    rng = numpy.random.RandomState(4)
+    xy = rng.uniform(-10 * pl, 10 * pl, (30, 2))
+    sets = [range(12), range(12), [3, 1, 7], [7, 3, 1], [29, 1, 5], list(range(30)),
+            list(range(30))[::-1], range(12)]
+    inputs = [(0.011 * k, numpy.column_stack([xy[list(ids)], list(ids), numpy.ones(len(ids))]))
+              for k, ids in enumerate(sets)]
+    frames = list(scopyon_amd.generate_images(inputs, 2, config=product_config(ov),
+                                              rng=numpy.random.RandomState(6), full_output=True))
+    for (img, info), (cam, oinfo) in zip(frames, _oracle_frames(ov, inputs, 6, nframes=2)):
+        numpy.testing.assert_allclose(info['expectation'], cam[:, :, 0], rtol=1e-10)
+        assert numpy.array_equal(img.as_array(), cam[:, :, 1])
+        st, ost = info['fluorescence_states'], oinfo['fluorescence_states']
+        assert list(st) == list(ost)
+        for m in ost:
+            assert st[m] == pytest.approx(ost[m], rel=1e-12, abs=0)
+        for m in oinfo['true_data']:
+            numpy.testing.assert_allclose(info['true_data'][m], oinfo['true_data'][m], rtol=1e-12)
+    bad = numpy.column_stack([xy, numpy.full(30, numpy.nan), numpy.ones(30)])
+    with pytest.raises(ValueError):
+        list(scopyon_amd.generate_images([(0.0, bad)], 1, config=product_config(ov),
+                                         rng=numpy.random.RandomState(6)))
+
+
 def test_form_image_errors(gpu):
     import scopyon_amd
     cfg = product_config({'detector': {'image_size': [8, 8]}})
