@@ -1116,7 +1116,8 @@ sep_gemm_kernel(SepArgs A) {
 #pragma unroll
             for (int k = 0; k < 4; ++k) C.q[k] = src[k];
             C.scale = i < ns ? (fax ? 1.0f : em.z) : 0.0f;
-            C.dst = (blk + fax * SG_BLOCK + fhb * 8 + (fax ? org >> 16 : (int)(short)org)) * 16 + fk;
+            C.dst = (blk + fax * SG_BLOCK + fhb * 8 + (fax ? org >> 16 : (int)(short)org)) * 16 +
+                    (DT == 0 ? (fk & 1) * 8 + (fk >> 1) : fk);
         };
         auto add = [&](const Chunk& C) {
             float v[8];
@@ -1139,7 +1140,9 @@ sep_gemm_kernel(SepArgs A) {
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            // lane (m, half): pixel m of the emitters 8 half .. 8 half + 7
+            // lane (m, half): pixel m of the emitters 8 half .. 8 half + 7; with float32
+            // operands of the even (half 0) or the odd ones, so that the chunk's emitters
+            // are added in list order
             if constexpr (DT == 0) {
                 const float4* pa = reinterpret_cast<const float4*>(&blkA[m][half * 8]);
                 const float4* pb = reinterpret_cast<const float4*>(&blkB[m][half * 8]);
