@@ -689,17 +689,24 @@ struct BwdTileArgs {
     int xcd;             // 1: workgroups map to tiles by smx::xcd_tile
 };
 
-__global__ void __launch_bounds__(BT_THREADS) gauss_backward_tile_kernel(BwdTileArgs A) {
+// Row stride of the staged window: the halo (TS + 2 R columns) with R columns
+// before it and what a 16-slot window reaches past it, zero off the frame, so
+// that every lane reads its four columns unclamped.  The row factors of a window
+// stay in the four lanes of its emitter and reach the others by DPP quad
+// broadcasts inside the multiply-adds (through LDS they cost a 16-byte read per
+// row and 17 KB, which held the CU to 16 waves; 64 x 256^2 with 5,000 emitters
+// each: 49 us so, 39 us now, with registers for 6 waves a SIMD; 41.9 with 4, 44.3
+// with 7).
+constexpr int BT_STRIDE = 64;
+static_assert(TS - 1 + 2 * 7 + GB <= BT_STRIDE, "window reach");
+
+__global__ void __launch_bounds__(BT_THREADS, 6) gauss_backward_tile_kernel(BwdTileArgs A) {
     // the tile's window of dL/dmu with R zero guard rows above and below
     // (rows of an off-frame window centre past the window are off the frame)
-    __shared__ float s_g[(HALO_MAX + 14) * HALO_MAX];
+    __shared__ float s_g[(HALO_MAX + 14) * BT_STRIDE];
     __shared__ float4 s_em[BT_THREADS];       // owned emitters: x, y, z, I
     __shared__ int s_own[BT_THREADS];
     __shared__ double s_gs[BT_THREADS];
-    // per emitter of a round, window row k: G, dG/dx, dG/dsigma
-    // (a float4 per row: one 16-byte read; one padding entry per group puts
-    // the 16 groups of a wave on distinct banks)
-    __shared__ float4 s_rowf[BT_GROUPS][GB + 1];
     __shared__ int s_wcnt[BT_THREADS / 64];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int R = A.P.radius, W = 2 * R + 1;
@@ -746,21 +753,21 @@ __global__ void __launch_bounds__(BT_THREADS) gauss_backward_tile_kernel(BwdTile
 #pragma unroll
     for (int i = 0; i < SROWS; ++i) {
         const int r = wave + i * (BT_THREADS / 64);
-        const int pr = hr0 - R + r, pc = hc0 + lane;
-        const bool ok = lane < HS && r >= R && r < HS + R && pr >= 0 && pr < F.nw && pc >= 0 &&
-                        pc < F.nh;
+        const int pr = hr0 - R + r, pc = hc0 - R + lane;
+        const bool ok = lane >= R && lane < HS + R && r >= R && r < HS + R && pr >= 0 &&
+                        pr < F.nw && pc >= 0 && pc < F.nh;
         gv[i] = ok ? A.grad_mu[(size_t)F.pix_off + (size_t)pr * F.nh + pc] : 0.0f;
     }
 #pragma unroll
     for (int i = 0; i < SROWS; ++i) {
         const int r = wave + i * (BT_THREADS / 64);
-        if (lane < HS && r < HS + 2 * R) s_g[r * HS + lane] = gv[i];
+        if (r < HS + 2 * R) s_g[r * BT_STRIDE + lane] = gv[i];
     }
     if ((long long)begin + count > A.capacity) count = (int)max(0LL, A.capacity - begin);
     const int* list = A.list + begin;
     // four lanes per emitter: lane q of group grp holds window slots
-    // 4 q .. 4 q + 3 of both axes: the factors of its rows (into LDS) and of
-    // its columns (registers) from two 16-byte table loads per axis and
+    // 4 q .. 4 q + 3 of both axes: the factors of its rows and of its columns
+    // from two 16-byte table loads per axis and
     // quantity (one cache line per emitter, axis and quantity), then the
     // sums over all rows for its four columns
     const int grp = tid >> 2, q = tid & 3;
@@ -803,7 +810,6 @@ __global__ void __launch_bounds__(BT_THREADS) gauss_backward_tile_kernel(BwdTile
             const int su = table_slot(v.x - fxl, fu) + 4 * q, sv = table_slot(v.y - fyl, fv) + 4 * q;
             float gy[4], dgy[4], sgy[4];
             float ru[3][4];
-            int hcol[4];
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
                 const float4* tu = tab4 + ((c * TABLE_ENTRIES + su) >> 1);
@@ -818,43 +824,34 @@ __global__ void __launch_bounds__(BT_THREADS) gauss_backward_tile_kernel(BwdTile
 #pragma unroll
                 for (int i = 0; i < 4; ++i) (c == 0 ? gy : c == 1 ? dgy : sgy)[i] = rv[i];
             }
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (4 * q + i < W)
-                    s_rowf[grp][4 * q + i] = make_float4(ru[0][i], ru[1][i], ru[2][i], 0.0f);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                // a column outside the staged block (off the frame) or past
-                // the window reads a clamped cell and has zero factors
-                const int jj = 4 * q + i, hc = lv + jj - hc0;
-                const bool col_in = valid && jj < W && hc >= 0 && hc < HS;
-                gy[i] = col_in ? gy[i] : 0.0f;
-                dgy[i] = col_in ? dgy[i] : 0.0f;
-                sgy[i] = col_in ? sgy[i] : 0.0f;
-                hcol[i] = min(max(hc, 0), HS - 1);
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            // staged row of window row 0: lu - (hr0 - R) in [0, HS + R] for
-            // every owned emitter
-            const float* grow = s_g + (valid ? (lu - hr0 + R) : 0) * HS;
+            // staged row and column of the window's first pixel: both in [0, 31 + 2 R]
+            // for every owned emitter; slots past the window have zero factors
+            const float* grow = s_g + (lu - hr0 + R) * BT_STRIDE + (lv - hc0 + R) + 4 * q;
             float t1[4] = {0.0f, 0.0f, 0.0f, 0.0f}, t2[4] = {0.0f, 0.0f, 0.0f, 0.0f};
             float t3[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            auto rows = [&](auto lane4) {
+                // window rows 4 j .. 4 j + 3: factors held by lane j of the quad
+                constexpr int j = decltype(lane4)::value, bcast = j * 0x55;
 #pragma unroll
-            for (int k = 0; k < WMAX; ++k) {
-                if (k < W) {
-                    const float4 fk = s_rowf[grp][k];
-                    const float f0 = fk.x, f1 = fk.y, f2 = fk.z;
+                for (int i = 0; i < 4; ++i) {
+                    const int k = 4 * j + i;
+                    if (k >= WMAX || k >= W) break;
+                    const float f0 = smx::dpp_f32<bcast>(ru[0][i]);
+                    const float f1 = smx::dpp_f32<bcast>(ru[1][i]);
+                    const float f2 = smx::dpp_f32<bcast>(ru[2][i]);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float g = grow[k * HS + hcol[i]];
-                        t1[i] = fmaf(g, f0, t1[i]);
-                        t2[i] = fmaf(g, f1, t2[i]);
-                        t3[i] = fmaf(g, f2, t3[i]);
+                    for (int c = 0; c < 4; ++c) {
+                        const float g = grow[k * BT_STRIDE + c];
+                        t1[c] = fmaf(g, f0, t1[c]);
+                        t2[c] = fmaf(g, f1, t2[c]);
+                        t3[c] = fmaf(g, f2, t3[c]);
                     }
                 }
-            }
+            };
+            rows(std::integral_constant<int, 0>());
+            rows(std::integral_constant<int, 1>());
+            rows(std::integral_constant<int, 2>());
+            rows(std::integral_constant<int, 3>());
             float vI[4], vx[4], vy[4], vs[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -879,9 +876,6 @@ __global__ void __launch_bounds__(BT_THREADS) gauss_backward_tile_kernel(BwdTile
             const float gs = emitter_outputs(pI, px, py, ps, q == 0 ? ee : -1, valid, v.z, v.w,
                                              A.P.inv_depth, A.gx, A.gy, A.gz, A.gI);
             if (valid && q == 0) s_gs[o] = (double)gs;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
         __syncthreads();
         if (wave == 0) {

@@ -893,9 +893,10 @@ struct DetectArgs {
 // compact the entries that meet their quadrant (about 2 in 5 of a 32 px tile's)
 // before they clip them, from 128 staged entries: a list of 77 entries, the
 // headline batch's average, is then one round of ~31 footprints per wave
-// instead of two rounds of 64 and 13 (@C@).  One-wave tiles meet every entry,
-// and LUT footprints (56% of a tile's entries meet a quadrant) and their
-// registers leave the staging no room: 64 there.
+// instead of two rounds of 64 and 13 (the headline tile pass 320 us so, 300 us
+// now).  One-wave tiles meet every entry, and LUT footprints (56% of a tile's
+// entries meet a quadrant) and their registers leave the staging no room: 64
+// there.
 template <int QPW, int TAPS> constexpr bool compacts() { return QPW > 1 && TAPS == 1; }
 template <int QPW, int TAPS> constexpr int fchunk() { return compacts<QPW, TAPS>() ? 128 : 64; }
 
