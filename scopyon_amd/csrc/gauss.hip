@@ -1381,10 +1381,13 @@ int gauss_bin(int n, const float* x, const float* y, const float* z, const float
                                stream, n, x, y, frame_id, frames_dev, nframes, R, n_tiles,
                                ws.tile_begin, ws.tile_count, cs, ws.list, capacity, status_dev);
         SMX_CHECK_LAUNCH("gauss_bin_fill_kernel");
-        hipLaunchKernelGGL(smx::sort_long_lists_kernel, dim3(smx::LONG_SORT_BLOCKS),
-                           dim3(smx::LONG_SORT_THREADS), 0, stream, ws.long_tiles, ws.tile_begin,
-                           ws.list, capacity, status_dev);
-        SMX_CHECK_LAUNCH("sort_long_lists_kernel");
+        // no list is longer than the emitters are many
+        if (n > PSORT_CAP) {
+            hipLaunchKernelGGL(smx::sort_long_lists_kernel, dim3(smx::LONG_SORT_BLOCKS),
+                               dim3(smx::LONG_SORT_THREADS), 0, stream, ws.long_tiles,
+                               ws.tile_begin, ws.list, capacity, status_dev);
+            SMX_CHECK_LAUNCH("sort_long_lists_kernel");
+        }
     }
     return SMX_OK;
 }

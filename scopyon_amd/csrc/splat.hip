@@ -1719,10 +1719,13 @@ static int splat_run(int n, const double* u, const double* v, const double* w, c
                                    fov_id, fovs_dev, nfov, ext_half, n_tiles, ws.tile_begin,
                                    ws.tile_count, cs, ws.list, list_capacity, status_dev);
             SMX_CHECK_LAUNCH("bin_fill_kernel");
-            hipLaunchKernelGGL(smx::sort_long_lists_kernel, dim3(smx::LONG_SORT_BLOCKS),
-                               dim3(smx::LONG_SORT_THREADS), 0, stream, ws.long_tiles,
-                               ws.tile_begin, ws.list, list_capacity, status_dev);
-            SMX_CHECK_LAUNCH("sort_long_lists_kernel");
+            // no list is longer than the emitters are many
+            if (n > long_min) {
+                hipLaunchKernelGGL(smx::sort_long_lists_kernel, dim3(smx::LONG_SORT_BLOCKS),
+                                   dim3(smx::LONG_SORT_THREADS), 0, stream, ws.long_tiles,
+                                   ws.tile_begin, ws.list, list_capacity, status_dev);
+                SMX_CHECK_LAUNCH("sort_long_lists_kernel");
+            }
         }
     }
     if (!(stages & 2)) return SMX_OK;
