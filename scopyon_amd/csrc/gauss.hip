@@ -188,7 +188,7 @@ __global__ void __launch_bounds__(256) gauss_init_kernel(int nfov,
     __shared__ smx::TilesInitLds L;
     if ((int)blockIdx.x < tile_blocks) {
         smx::tiles_init_block(L, blockIdx.x, nfov, fovs, n_tiles, tile_count, cs, tile_fov,
-                              long_tiles);
+                              long_tiles, nullptr);
         return;
     }
     const int idx = ((int)blockIdx.x - tile_blocks) * blockDim.x + threadIdx.x;
@@ -1358,13 +1358,13 @@ int gauss_bin(int n, const float* x, const float* y, const float* z, const float
         // one workgroup scans the counters in place of compact + device scan
         hipLaunchKernelGGL(smx::scan_counts_kernel, dim3(1), dim3(smx::SCAN_THREADS), 0, stream,
                            ws.tile_count, cs, n_tiles + 1, ws.tile_begin, PSORT_CAP,
-                           ws.long_tiles);
+                           ws.long_tiles, smx::HeavyTiles{});
         SMX_CHECK_LAUNCH("scan_counts_kernel");
     } else {
         size_t cb = ws.cub_bytes;
         hipLaunchKernelGGL(smx::compact_counts_kernel, dim3((n_tiles + 1 + 255) / 256), dim3(256),
                            0, stream, ws.tile_count, cs, n_tiles + 1, ws.tile_dense, PSORT_CAP,
-                           ws.long_tiles);
+                           ws.long_tiles, smx::HeavyTiles{});
         SMX_CHECK_LAUNCH("compact_counts_kernel");
         if (smx::check_hip(hipcub::DeviceScan::ExclusiveSum(ws.cub_tmp, cb, ws.tile_dense,
                                                             ws.tile_begin, n_tiles + 1, stream),

@@ -58,15 +58,30 @@ __device__ inline void note_long(int* long_tiles, int long_min, int g, int count
     }
 }
 
+// Tiles with lists much longer than the average (more than `min` entries) are
+// noted the same way, up to `cap` of them (list[0] counts on past it): the tile
+// pass starts them first.
+struct HeavyTiles {
+    int* list;   // NULL: none are noted; list[0] = how many, list[1 ..] = the tiles
+    int min, cap;
+};
+__device__ inline void note_heavy(const HeavyTiles& H, int g, int count) {
+    if (H.list && count > H.min) {
+        const int k = atomicAdd(H.list, 1);
+        if (k < H.cap) H.list[1 + k] = g;
+    }
+}
+
 // Dense copy of the counters for the scan: dense[g] = counts[g * cs].
 __global__ void compact_counts_kernel(const int* __restrict__ counts, int cs, int n,
                                       int* __restrict__ dense, int long_min,
-                                      int* __restrict__ long_tiles) {
+                                      int* __restrict__ long_tiles, HeavyTiles heavy) {
     const int g = blockIdx.x * blockDim.x + threadIdx.x;
     if (g < n) {
         const int c = counts[(size_t)g * cs];
         dense[g] = c;
         note_long(long_tiles, long_min, g, c);
+        note_heavy(heavy, g, c);
     }
 }
 
@@ -88,14 +103,16 @@ __global__ void __launch_bounds__(SCAN_THREADS) scan_counts_kernel(const int* __
                                                                   int cs, int n,
                                                                   int* __restrict__ begin,
                                                                   int long_min,
-                                                                  int* __restrict__ long_tiles) {
+                                                                  int* __restrict__ long_tiles,
+                                                                  HeavyTiles heavy) {
     constexpr int NW = SCAN_THREADS / 64;
     static_assert(NW == 16, "one DPP row of 16 lanes scans the wave totals");
     __shared__ int s_wave[SCAN_ROWS][NW];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    // the long-list count starts at zero here (a binning that skips the
+    // the counts of noted tiles start at zero here (a binning that skips the
     // counter initialisation relies on it)
     if (t == 0 && long_tiles) long_tiles[0] = 0;
+    if (t == 0 && heavy.list) heavy.list[0] = 0;
     __syncthreads();
     int carry = 0;   // sum of the rows before
     for (int base = 0; base < n; base += SCAN_THREADS * SCAN_ROWS) {
@@ -108,7 +125,10 @@ __global__ void __launch_bounds__(SCAN_THREADS) scan_counts_kernel(const int* __
 #pragma unroll
         for (int r = 0; r < SCAN_ROWS; ++r) {
             const int g = base + r * SCAN_THREADS + t;
-            if (g < n) note_long(long_tiles, long_min, g, c[r]);
+            if (g < n) {
+                note_long(long_tiles, long_min, g, c[r]);
+                note_heavy(heavy, g, c[r]);
+            }
             incl[r] = c[r];
         }
 #pragma unroll
@@ -150,7 +170,8 @@ __device__ inline void tiles_init_block(TilesInitLds& L, int block, int nfov,
                                         const smx_fov_t* __restrict__ fovs, int n_tiles,
                                         int* __restrict__ tile_count, int cs,
                                         int* __restrict__ tile_fov,
-                                        int* __restrict__ long_tiles) {
+                                        int* __restrict__ long_tiles,
+                                        int* __restrict__ heavy_tiles) {
     const int staged = nfov < TILES_INIT_FOVS ? nfov : TILES_INIT_FOVS;
     if (threadIdx.x == 0) L.unsorted = 0;
     __syncthreads();
@@ -167,6 +188,7 @@ __device__ inline void tiles_init_block(TilesInitLds& L, int block, int nfov,
     tile_count[(size_t)g * cs] = 0;
     if (g == n_tiles) {
         if (long_tiles) long_tiles[0] = 0;
+        if (heavy_tiles) heavy_tiles[0] = 0;
         return;
     }
     int owner = -1;
@@ -195,9 +217,11 @@ __global__ void __launch_bounds__(256) tiles_init_kernel(int nfov,
                                                          const smx_fov_t* __restrict__ fovs,
                                                          int n_tiles, int* __restrict__ tile_count,
                                                          int cs, int* __restrict__ tile_fov,
-                                                         int* __restrict__ long_tiles) {
+                                                         int* __restrict__ long_tiles,
+                                                         int* __restrict__ heavy_tiles) {
     __shared__ TilesInitLds L;
-    tiles_init_block(L, blockIdx.x, nfov, fovs, n_tiles, tile_count, cs, tile_fov, long_tiles);
+    tiles_init_block(L, blockIdx.x, nfov, fovs, n_tiles, tile_count, cs, tile_fov, long_tiles,
+                     heavy_tiles);
 }
 
 // Ascending bitonic sort of n_pow2 ints in LDS by the whole workgroup.

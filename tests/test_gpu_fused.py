@@ -172,3 +172,33 @@ def test_self_listed_tiles_equal_binned(gpu, nfov, n, kind):
     assert frames[0][0].abs().sum() > 0
     for photons, adc in frames[1:]:
         assert torch.equal(photons, frames[0][0]) and torch.equal(adc, frames[0][1])
+
+
+@pytest.mark.parametrize('clustered,spread', [(0, 1.0), (6000, 0.08), (6000, 0.4), (60000, 0.5)])
+def test_heavy_tiles_first(gpu, clustered, spread):
+    """Launches of 4,096 tiles and more start their heaviest tiles first, as many as
+    their list holds (256 of 4,099 here: none are heavy, some, or more than it
+    holds); fewer, larger tiles note none.  Photons and counts are the same bits."""
+    from scopyon_amd.batched import BatchedSimulator
+    ov = {'detector': {'image_size': [64, 64], 'exposure_time': 0.033},
+          'magnification': 100.0, 'effects': {'photo_bleaching': {'switch': False}}}
+    shapes = [(1024, 1024), (33, 16)]
+    rng = numpy.random.RandomState(clustered)
+    n = 500 + clustered // 2
+    x = rng.uniform(-512, 512, (2, 2 * n)) * 1.6e-7
+    x[:, :clustered] *= spread
+    fov = numpy.zeros(2 * n, dtype=numpy.int32)
+    fov[-100:] = 1
+    frames = []
+    for side in (16, 32, 64):
+        sim = BatchedSimulator(product_config(ov), shapes, n, dt=0.033, seed=5, tile_side=side,
+                               keep_photons=True, psf='table', table_precision='folded')
+        sim.fov_id.copy_(torch.as_tensor(fov))
+        sim.set_positions(numpy.zeros(2 * n), x[0], x[1])
+        for step in range(2):
+            sim.splat_detect()
+            frames.append((sim.photons.clone(), sim.adc.clone()))
+        assert sim.status() == 0
+    assert frames[0][0].abs().sum() > 0
+    for photons, adc in frames[1:]:
+        assert torch.equal(photons, frames[0][0]) and torch.equal(adc, frames[0][1])
