@@ -479,7 +479,9 @@ __device__ inline void wave_sort_list(const int* src, int count, int lane, int* 
 }
 
 // In-place sort of the noted long tile lists (see note_long), up to
-// LONG_SORT_CAP entries each: every wave sorts 1024-entry runs in registers
+// LONG_SORT_CAP entries each: up to 2048 entries through buckets (64 lists of
+// ~1,650 entries among 256 uneven frames: step 933 us with the merge, 923 so);
+// longer ones by merging: every wave sorts 1024-entry runs in registers
 // (wave_sort), then the runs are merged pairwise in LDS -- an entry's place in
 // the merged run is its index in its own run plus its rank in the partner run
 // (lower bound from the left run, upper bound from the right one, so the INT_MAX
@@ -505,6 +507,12 @@ __global__ void __launch_bounds__(LONG_SORT_THREADS) sort_long_lists_kernel(
             continue;
         }
         int* L = list + begin;
+        if (count <= 4 * LONG_SORT_THREADS) {
+            bucket_sort<LONG_SORT_THREADS, 4>(L, count, buf[0], buf[1]);
+            for (int i = threadIdx.x; i < count; i += blockDim.x) L[i] = buf[1][i];
+            __syncthreads();
+            continue;
+        }
         const int nch = (count + 1023) >> 10;
         for (int c = wave; c < nch; c += LONG_SORT_THREADS / 64)
             wave_sort<16>(L + c * 1024, min(1024, count - c * 1024), lane, buf[0] + c * 1024);
