@@ -1234,172 +1234,173 @@ splat_phase_kernel(FastArgs A, DetectArgs D) {
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             }
             for (int hb = 0; hb < (LP::COMPACT ? nh : 1); hb += 64) {
-            // footprint rectangle of this lane's entry `ix` inside the quadrant:
-            // origin (rr0, cc0) in the quadrant, width W, `area` pixels in np
-            // parts, kq = table element of its first pixel
-            const bool mine = hb + lane < nh;
-            const int ix = LP::COMPACT ? (int)s_idx[min(hb + lane, nh - 1)] : lane;
-            int np = 0, W = 1, area = 0, rr0 = 0, cc0 = 0, su = 0, sv = 0;
-            long long kq = 0;
-            bool irr = false;
-            if (mine && s_flags[ix] != 2) {
-                const int4 g = s_geo[ix];
-                const int r0 = max(g.x, qr0), r1 = min(g.x + g.z, qr0 + qh);
-                const int c0 = max(g.y, qc0), c1 = min(g.y + g.w, qc0 + qw);
-                if (r1 > r0 && c1 > c0) {
-                    const int2 st = s_str[ix];
-                    W = c1 - c0;
-                    area = (r1 - r0) * W;
-                    np = (area + 63) >> 6;
-                    irr = s_flags[ix] == 1;
-                    rr0 = r0 - qr0;
-                    cc0 = c0 - qc0;
-                    su = st.x;
-                    sv = st.y;
-                    kq = s_ko[ix] + (long long)(r0 - g.x) * su + (long long)(c0 - g.y) * sv;
+                // footprint rectangle of this lane's entry `ix` inside the quadrant:
+                // origin (rr0, cc0) in the quadrant, width W, `area` pixels in np
+                // parts, kq = table element of its first pixel
+                const bool mine = hb + lane < nh;
+                const int ix = LP::COMPACT ? (int)s_idx[min(hb + lane, nh - 1)] : lane;
+                int np = 0, W = 1, area = 0, rr0 = 0, cc0 = 0, su = 0, sv = 0;
+                long long kq = 0;
+                bool irr = false;
+                if (mine && s_flags[ix] != 2) {
+                    const int4 g = s_geo[ix];
+                    const int r0 = max(g.x, qr0), r1 = min(g.x + g.z, qr0 + qh);
+                    const int c0 = max(g.y, qc0), c1 = min(g.y + g.w, qc0 + qw);
+                    if (r1 > r0 && c1 > c0) {
+                        const int2 st = s_str[ix];
+                        W = c1 - c0;
+                        area = (r1 - r0) * W;
+                        np = (area + 63) >> 6;
+                        irr = s_flags[ix] == 1;
+                        rr0 = r0 - qr0;
+                        cc0 = c0 - qc0;
+                        su = st.x;
+                        sv = st.y;
+                        kq = s_ko[ix] + (long long)(r0 - g.x) * su + (long long)(c0 - g.y) * sv;
+                    }
                 }
-            }
-            const bool any_irregular = __ballot(irr) != 0;
-            const int incl = smx::wave_incl_scan(np);
-            const int first = incl - np;   // this emitter's parts: [first, incl) in list order
-            const int total = __builtin_amdgcn_readlane(incl, 63);
+                const bool any_irregular = __ballot(irr) != 0;
+                const int incl = smx::wave_incl_scan(np);
+                const int first = incl - np;   // this emitter's parts: [first, incl) in list order
+                const int total = __builtin_amdgcn_readlane(incl, 63);
 
-            if (any_irregular) {
-                // rare (a float64 tie in a cell boundary): one part at a time, in
-                // order, flagged emitters integrated through the SAT
-                for (int b = 0; b < total; ++b) {
-                    const int c = __popcll(__ballot(incl <= b));   // emitter lane owning part b
-                    const int p = b - __shfl(first, c);
-                    const int Wc = __shfl(W, c), ar = __shfl(area, c);
-                    const int rc = __shfl(rr0, c), cc = __shfl(cc0, c);
-                    const int suc = __shfl(su, c), svc = __shfl(sv, c);
-                    const long long kqc = __shfl(kq, c);
-                    const int xc = __shfl(ix, c);
-                    const int idx = p * 64 + lane;
-                    if (idx >= ar) continue;
-                    const int row = idx / Wc, col = idx - row * Wc;
-                    double val;
-                    if (s_flags[xc] == 1) {
-                        val = sat_pixel(A, F, s_e[xc], s_w[xc], qr0 + rc + row, qc0 + cc + col, 0.0);
-                    } else {
-                        val = (double)smx::gload((const KT*)A.Kraw + kqc + (long long)row * suc +
-                                                 (long long)col * svc) *
-                              s_w[xc];
-                    }
-                    lds_add(acc + (rc + row) * AS + cc + col, val);
-                }
-            } else {
-                PartRec* pr = s_pr[wave];
-                double* pw = s_pw[wave];
-                // float tables: the weight in float32 too, the product converted
-                // to float64 for the add (contribution within ~3 2^-24 relative)
-                constexpr bool F32W = std::is_same<KT, float>::value && TAPS == 1;
-                float* pwf = reinterpret_cast<float*>(pw);
-                float4* pc = s_pc[wave];
-                const int magic = (65536 + W - 1) / W;
-                const double w = mine ? s_w[ix] : 0.0;
-                // LUT mode: bilinear weights of the four phase taps, times w
-                float4 cw = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (TAPS == 4 && mine) {
-                    const unsigned fr = s_frac[ix];
-                    const float fu = (float)(fr & 0xffffu) * (1.0f / 65535.0f);
-                    const float fv = (float)(fr >> 16) * (1.0f / 65535.0f);
-                    const float wf = (float)w;
-                    cw = make_float4(((1.0f - fu) * (1.0f - fv)) * wf, ((1.0f - fu) * fv) * wf,
-                                     (fu * (1.0f - fv)) * wf, (fu * fv) * wf);
-                }
-                const long long kb = kq * (long long)sizeof(KT);
-                const unsigned long long ka = (unsigned long long)(kbase + kb);
-                const int pix = acc_off + (rr0 * AS + cc0) * 8;
-                for (int rb = 0; rb < total; rb += PMAX) {
-                    // this round's parts [rb, rb + PMAX), then null records up to
-                    // a whole number of NS groups (no lane valid, table offset 0)
-                    for (int p = 0; p < np; ++p) {
-                        const int pos = first + p - rb;
-                        if ((unsigned)pos >= (unsigned)PMAX) continue;
-                        const int lim = min(64, area - p * 64);
-                        PartRec& R = pr[pos];
-                        R.kq = O32 ? (int)(unsigned)kb : (int)(unsigned)ka;
-                        R.magic_lim = magic | (lim << 24);
-                        R.dk = (su - W * sv) * (int)sizeof(KT);
-                        R.p64 = p * 64;
-                        R.da = (AS - W) * 8;
-                        R.sv = sv * (int)sizeof(KT);
-                        R.pix = pix;
-                        R.kq_hi = O32 ? 0 : (int)(unsigned)(ka >> 32);
-                        if (TAPS == 4) pc[pos] = cw;
-                        else if (F32W) pwf[pos] = (float)w;
-                        else pw[pos] = w;
-                    }
-                    const int cnt = min(PMAX, total - rb);
-                    const int cntp = (cnt + NS - 1) & ~(NS - 1);
-                    if (lane >= cnt && lane < cntp) {
-                        PartRec& R = pr[lane];
-                        R.kq = O32 ? 0 : (int)(unsigned)(unsigned long long)kbase;
-                        R.magic_lim = 0;
-                        R.dk = 0;
-                        R.p64 = 0;
-                        R.da = 0;
-                        R.sv = 0;
-                        R.pix = 0;
-                        R.kq_hi = O32 ? 0 : (int)(unsigned)((unsigned long long)kbase >> 32);
-                        if (TAPS == 4) pc[lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                        else if (F32W) pwf[lane] = 0.0f;
-                        else pw[lane] = 0.0;
-                    }
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                    for (int b = 0; b < cntp; b += NS) {
-                        KT kv[NS];
-                        float4 kc[NS];   // LUT cell: the four taps of a pixel
-                        double wv[NS];
-                        float wf[NS];
-                        unsigned la[NS];
-#pragma unroll
-                        for (int s = 0; s < NS; ++s) {
-                            const PartRec& R = pr[b + s];
-                            const int4 h = *(const int4*)&R.kq;   // kq, magic_lim, dk, p64
-                            const int4 g = *(const int4*)&R.da;   // da, sv, pix, kq_hi
-                            if (F32W) wf[s] = pwf[b + s];
-                            else if (TAPS == 1) wv[s] = pw[b + s];
-                            const unsigned idx = (unsigned)lane + (unsigned)h.w;
-                            const bool ok = lane24 < (unsigned)h.y;
-                            const int row = (int)(__umul24(idx, (unsigned)h.y) >> 16);
-                            const char* kp;
-                            if (O32) {
-                                int off = __mul24(row, h.z) + (__mul24((int)idx, g.y) + h.x);
-                                off = ok ? off : 0;
-                                kp = kbase + (unsigned)off;
-                            } else {
-                                int off = __mul24(row, h.z) + __mul24((int)idx, g.y);
-                                off = ok ? off : 0;
-                                kp = (const char*)(((unsigned long long)(unsigned)g.w << 32) |
-                                                   (unsigned)h.x) + off;
-                            }
-                            if (TAPS == 4) kc[s] = smx::gload4((const float*)kp);
-                            else kv[s] = smx::gload((const KT*)kp);
-                            const unsigned l = (unsigned)__mul24(row, g.x) + ((unsigned)g.z + (idx << 3));
-                            la[s] = ok ? l : spill;
+                if (any_irregular) {
+                    // rare (a float64 tie in a cell boundary): one part at a time, in
+                    // order, flagged emitters integrated through the SAT
+                    for (int b = 0; b < total; ++b) {
+                        const int c = __popcll(__ballot(incl <= b));   // emitter lane owning part b
+                        const int p = b - __shfl(first, c);
+                        const int Wc = __shfl(W, c), ar = __shfl(area, c);
+                        const int rc = __shfl(rr0, c), cc = __shfl(cc0, c);
+                        const int suc = __shfl(su, c), svc = __shfl(sv, c);
+                        const long long kqc = __shfl(kq, c);
+                        const int xc = __shfl(ix, c);
+                        const int idx = p * 64 + lane;
+                        if (idx >= ar) continue;
+                        const int row = idx / Wc, col = idx - row * Wc;
+                        double val;
+                        if (s_flags[xc] == 1) {
+                            val = sat_pixel(A, F, s_e[xc], s_w[xc], qr0 + rc + row,
+                                            qc0 + cc + col, 0.0);
+                        } else {
+                            val = (double)smx::gload((const KT*)A.Kraw + kqc + (long long)row * suc +
+                                                     (long long)col * svc) *
+                                  s_w[xc];
                         }
+                        lds_add(acc + (rc + row) * AS + cc + col, val);
+                    }
+                } else {
+                    PartRec* pr = s_pr[wave];
+                    double* pw = s_pw[wave];
+                    // float tables: the weight in float32 too, the product converted
+                    // to float64 for the add (contribution within ~3 2^-24 relative)
+                    constexpr bool F32W = std::is_same<KT, float>::value && TAPS == 1;
+                    float* pwf = reinterpret_cast<float*>(pw);
+                    float4* pc = s_pc[wave];
+                    const int magic = (65536 + W - 1) / W;
+                    const double w = mine ? s_w[ix] : 0.0;
+                    // LUT mode: bilinear weights of the four phase taps, times w
+                    float4 cw = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                    if (TAPS == 4 && mine) {
+                        const unsigned fr = s_frac[ix];
+                        const float fu = (float)(fr & 0xffffu) * (1.0f / 65535.0f);
+                        const float fv = (float)(fr >> 16) * (1.0f / 65535.0f);
+                        const float wf = (float)w;
+                        cw = make_float4(((1.0f - fu) * (1.0f - fv)) * wf, ((1.0f - fu) * fv) * wf,
+                                         (fu * (1.0f - fv)) * wf, (fu * fv) * wf);
+                    }
+                    const long long kb = kq * (long long)sizeof(KT);
+                    const unsigned long long ka = (unsigned long long)(kbase + kb);
+                    const int pix = acc_off + (rr0 * AS + cc0) * 8;
+                    for (int rb = 0; rb < total; rb += PMAX) {
+                        // this round's parts [rb, rb + PMAX), then null records up to
+                        // a whole number of NS groups (no lane valid, table offset 0)
+                        for (int p = 0; p < np; ++p) {
+                            const int pos = first + p - rb;
+                            if ((unsigned)pos >= (unsigned)PMAX) continue;
+                            const int lim = min(64, area - p * 64);
+                            PartRec& R = pr[pos];
+                            R.kq = O32 ? (int)(unsigned)kb : (int)(unsigned)ka;
+                            R.magic_lim = magic | (lim << 24);
+                            R.dk = (su - W * sv) * (int)sizeof(KT);
+                            R.p64 = p * 64;
+                            R.da = (AS - W) * 8;
+                            R.sv = sv * (int)sizeof(KT);
+                            R.pix = pix;
+                            R.kq_hi = O32 ? 0 : (int)(unsigned)(ka >> 32);
+                            if (TAPS == 4) pc[pos] = cw;
+                            else if (F32W) pwf[pos] = (float)w;
+                            else pw[pos] = w;
+                        }
+                        const int cnt = min(PMAX, total - rb);
+                        const int cntp = (cnt + NS - 1) & ~(NS - 1);
+                        if (lane >= cnt && lane < cntp) {
+                            PartRec& R = pr[lane];
+                            R.kq = O32 ? 0 : (int)(unsigned)(unsigned long long)kbase;
+                            R.magic_lim = 0;
+                            R.dk = 0;
+                            R.p64 = 0;
+                            R.da = 0;
+                            R.sv = 0;
+                            R.pix = 0;
+                            R.kq_hi = O32 ? 0 : (int)(unsigned)((unsigned long long)kbase >> 32);
+                            if (TAPS == 4) pc[lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                            else if (F32W) pwf[lane] = 0.0f;
+                            else pw[lane] = 0.0;
+                        }
+                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
+                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                        for (int b = 0; b < cntp; b += NS) {
+                            KT kv[NS];
+                            float4 kc[NS];   // LUT cell: the four taps of a pixel
+                            double wv[NS];
+                            float wf[NS];
+                            unsigned la[NS];
 #pragma unroll
-                        for (int s = 0; s < NS; ++s) {
-                            if (TAPS == 4) {
-                                const float4 c = pc[b + s];
-                                const float val = ((c.x * kc[s].x + c.y * kc[s].y) + c.z * kc[s].z) +
-                                                  c.w * kc[s].w;
-                                lds_add((double*)((char*)s_acc + la[s]), (double)val);
-                            } else {
-                                lds_add((double*)((char*)s_acc + la[s]),
-                                        F32W ? (double)((float)kv[s] * wf[s]) : (double)kv[s] * wv[s]);
+                            for (int s = 0; s < NS; ++s) {
+                                const PartRec& R = pr[b + s];
+                                const int4 h = *(const int4*)&R.kq;   // kq, magic_lim, dk, p64
+                                const int4 g = *(const int4*)&R.da;   // da, sv, pix, kq_hi
+                                if (F32W) wf[s] = pwf[b + s];
+                                else if (TAPS == 1) wv[s] = pw[b + s];
+                                const unsigned idx = (unsigned)lane + (unsigned)h.w;
+                                const bool ok = lane24 < (unsigned)h.y;
+                                const int row = (int)(__umul24(idx, (unsigned)h.y) >> 16);
+                                const char* kp;
+                                if (O32) {
+                                    int off = __mul24(row, h.z) + (__mul24((int)idx, g.y) + h.x);
+                                    off = ok ? off : 0;
+                                    kp = kbase + (unsigned)off;
+                                } else {
+                                    int off = __mul24(row, h.z) + __mul24((int)idx, g.y);
+                                    off = ok ? off : 0;
+                                    kp = (const char*)(((unsigned long long)(unsigned)g.w << 32) |
+                                                       (unsigned)h.x) + off;
+                                }
+                                if (TAPS == 4) kc[s] = smx::gload4((const float*)kp);
+                                else kv[s] = smx::gload((const KT*)kp);
+                                const unsigned l = (unsigned)__mul24(row, g.x) + ((unsigned)g.z + (idx << 3));
+                                la[s] = ok ? l : spill;
+                            }
+#pragma unroll
+                            for (int s = 0; s < NS; ++s) {
+                                if (TAPS == 4) {
+                                    const float4 c = pc[b + s];
+                                    const float val = ((c.x * kc[s].x + c.y * kc[s].y) + c.z * kc[s].z) +
+                                                      c.w * kc[s].w;
+                                    lds_add((double*)((char*)s_acc + la[s]), (double)val);
+                                } else {
+                                    lds_add((double*)((char*)s_acc + la[s]),
+                                            F32W ? (double)((float)kv[s] * wf[s]) : (double)kv[s] * wv[s]);
+                                }
                             }
                         }
+                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
+                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
                     }
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
                 }
-            }
             }
         }
         __syncthreads();
