@@ -929,7 +929,7 @@ __device__ __forceinline__ double sat_pixel(const FastArgs& A, const smx_fov_t& 
 // quadrant and splits each rectangle into 64-pixel parts (lane = pixel of the
 // rectangle, so no lane idles outside it).  The parts go to LDS as decoded
 // records, up to PMAX per round, padded with null records to whole groups of
-// nslot; per group the lanes issue nslot table loads at once (24-bit
+// NSLOT; per group the lanes issue NSLOT table loads at once (24-bit
 // multiply-adds on uniform record fields, byte offsets from the table base),
 // then add the contributions into the wave's LDS accumulator part by part in
 // list order, with no branch: lanes outside a part add into their own spill
@@ -942,10 +942,7 @@ __device__ __forceinline__ double sat_pixel(const FastArgs& A, const smx_fov_t& 
 // rows of a narrow part share banks, 17 spreads them (measured: 17 is the
 // fastest of 16, 17, 18, 20 and 24 for 16 x 16 quadrants).
 template <int QS> constexpr int acc_stride() { return QS + 1; }
-// 64-pixel parts in flight per wave (a round's parts are padded to a multiple):
-// 8 in tiles of several quadrants, 4 in one-wave tiles (256 uneven FOVs 936 ->
-// 931 us) and with LUT entries, four registers each (1024^2 frame 440 -> 433 us).
-template <int QPW, int TAPS> constexpr int nslot() { return QPW > 1 && TAPS == 1 ? 8 : 4; }
+constexpr int NSLOT = 8;          // 64-pixel parts in flight per wave
 // tile list sorted in LDS: 2048 entries, 1024 for one-wave tiles
 template <int QPW> constexpr int psort_cap() { return QPW == 1 ? 1024 : 2048; }
 
@@ -966,10 +963,7 @@ struct __align__(16) PartRec {
     int pix;         // accumulator byte offset of the rectangle's first pixel
     int kq_hi;       // high half of the byte address (64-bit form)
 };
-// parts per wave per round (one lane writes each padding record): 64, 32 in
-// one-wave tiles, whose LDS bounds the waves on a CU (9.7 -> 8.4 KB a wave, 256
-// uneven FOVs 931 -> 926 us)
-template <int QPW> constexpr int pmax() { return QPW == 1 ? 32 : 64; }
+constexpr int PMAX = 64;          // parts per wave per round (one lane writes each padding record)
 // waves per SIMD the register allocation leaves room for: 6 (<= 80 VGPRs; a
 // 32-pixel tile's block takes 22.5 KB of LDS, so 7 fit a CU; 7 waves would
 // spill)
@@ -985,7 +979,7 @@ template <int QPW> constexpr int pmax() { return QPW == 1 ? 32 : 64; }
 template <int QPW, bool DET, int TAPS, int QS>
 struct SplatLds {
     static constexpr int AS = acc_stride<QS>();
-    static constexpr int WPT = QPW * QPW, TSZ = QS * QPW, ACC = QS * AS, PMAX = pmax<QPW>();
+    static constexpr int WPT = QPW * QPW, TSZ = QS * QPW, ACC = QS * AS;
     // accumulators, then one spill slot per lane shared by the waves (lanes
     // outside a part add there: no branch per part, the slots are never read);
     // before the accumulators are cleared the same space sorts the tile list
@@ -1039,11 +1033,10 @@ splat_phase_kernel(FastArgs A, DetectArgs D) {
     __shared__ int s_list[SCAN ? SCAN_N : 1];
     __shared__ int s_hits[SCAN ? 2 * LP::WPT : 1];
     constexpr int AS = LP::AS;
-    // 64-pixel parts in flight per group: NS table loads (one 16-byte cell
+    // 64-pixel parts in flight per group: NSLOT table loads (one 16-byte cell
     // entry per part in LUT mode)
-    constexpr int NS = nslot<QPW, TAPS>();
+    constexpr int NS = NSLOT;
     constexpr int WPT = LP::WPT, TSZ = LP::TSZ, PSORT_CAP = psort_cap<QPW>();
-    constexpr int PMAX = LP::PMAX;
     constexpr int ACC = LP::ACC, ACCN = LP::ACCN;
     __shared__ __align__(16) char s_lds[LP::BYTES];
     double* const s_acc = (double*)s_lds;
