@@ -1120,6 +1120,12 @@ sep_gemm_kernel(SepArgs A) {
                 v[2 * i] = fmaf(C.f, C.q[i].y, C.q[i].x) * C.scale;
                 v[2 * i + 1] = fmaf(C.f, C.q[i].w, C.q[i].z) * C.scale;
             }
+            // the product is rounded to float32 before it becomes a float16 operand
+            // (left alone, multiply and conversion become one v_fma_mixlo_f16)
+            if constexpr (DT == 1) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) asm("" : "+v"(v[i]));
+            }
             // zero both blocks, then the windows
             float4* const zero = reinterpret_cast<float4*>(blkA[0]);
             constexpr int Z = TS * 16 * (int)sizeof(E) / 16 / 64;   // 16-byte stores a lane
