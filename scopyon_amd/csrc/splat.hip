@@ -1489,10 +1489,10 @@ struct SplatWorkspace {
 // eighth of the launch.  A tile of a dense frame or cluster runs for many times
 // the average; met in its turn near the end it outlives all others (256 uneven
 // frames, lists of 58 entries on average and 1,650 in the densest frame: step
-// 1,019 us in turn, 933 so; over 6 times the average, up to 1 / 32 of the tiles:
-// 10 us more).  Where no tile is heavy the idle workgroups cost 0.5% (64 like
-// frames: 345.5 and 347.3 us).  Launches of fewer tiles than start together
-// (5,000 one-wave workgroups) gain nothing and note none.
+// 1,023 us in turn, 937 so; over 6 times the average, up to 1 / 32 of the tiles:
+// 10 us more).  Where no tile is heavy the idle workgroups cost nothing that
+// shows (64 like frames: 347.3 us both ways).  Launches of fewer tiles than
+// start together (5,000 one-wave workgroups) gain nothing and note none.
 constexpr int HEAVY_TIMES = 3, HEAVY_TILES = 4096;
 int heavy_cap(int n_tiles) { return n_tiles >= HEAVY_TILES ? n_tiles / 16 & ~(smx::NXCD - 1) : 0; }
 

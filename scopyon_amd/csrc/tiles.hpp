@@ -480,7 +480,8 @@ __device__ inline void wave_sort_list(const int* src, int count, int lane, int* 
 
 // In-place sort of the noted long tile lists (see note_long), up to
 // LONG_SORT_CAP entries each: up to 2048 entries through buckets (64 lists of
-// ~1,650 entries among 256 uneven frames: step 933 us with the merge, 923 so);
+// ~1,650 entries among 256 uneven frames: 10 us less than with the merge, of a
+// step of 0.94 ms);
 // longer ones by merging: every wave sorts 1024-entry runs in registers
 // (wave_sort), then the runs are merged pairwise in LDS -- an entry's place in
 // the merged run is its index in its own run plus its rank in the partner run
