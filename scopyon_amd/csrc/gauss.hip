@@ -301,7 +301,7 @@ __global__ void __launch_bounds__(smx::BIN_THREADS) gauss_bin_fill_kernel(
         }
     }
     __syncthreads();
-    smx::bin_claim(s_hist, wbase, tile_begin, tile_left, cs);
+    smx::bin_claim(s_hist, wbase, tile_left, cs);
     __syncthreads();
 #pragma unroll
     for (int e = 0; e < EPT; ++e) {
@@ -310,7 +310,7 @@ __global__ void __launch_bounds__(smx::BIN_THREADS) gauss_bin_fill_kernel(
         for (int q = 0; q < 4; ++q) {
             if (ent[e][q] < 0) continue;
             const int d = ent[e][q] >> 16, rank = ent[e][q] & 0xffff;
-            const long long at = (long long)s_hist[d] + rank;
+            const long long at = (long long)tile_begin[wbase + d] + s_hist[d] + rank;
             if (at < capacity) list[at] = i;
             else atomicOr(status, 2);
         }

@@ -152,7 +152,7 @@ __device__ inline void count_entries(const smx_fov_t& F, const TileRange& t, int
 // thread has an emitter with tile range t in FOV F).  Entries of a footprint
 // within 2 x 2 tiles of the window take an LDS rank, the block claims each
 // window tile's slots with one global atomic, and the entries are written at
-// that place + rank; other entries claim a slot each.
+// claim + rank; other entries claim a slot each.
 __device__ inline void fill_entries(bool in, int i, const smx_fov_t* F, const TileRange& t,
                                     int n_tiles, int* s_hist, int wbase,
                                     const int* __restrict__ tile_begin,
@@ -182,13 +182,13 @@ __device__ inline void fill_entries(bool in, int i, const smx_fov_t* F, const Ti
             }
     }
     __syncthreads();
-    smx::bin_claim(s_hist, wbase, tile_begin, tile_left, cs);
+    smx::bin_claim(s_hist, wbase, tile_left, cs);
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         if (ent[q] < 0) continue;
         const int d = ent[q] >> 16, rank = ent[q] & 0xffff;
-        const long long at = (long long)s_hist[d] + rank;
+        const long long at = (long long)tile_begin[wbase + d] + s_hist[d] + rank;
         if (at < capacity) list[at] = i;
         else atomicOr(status, 2);
     }

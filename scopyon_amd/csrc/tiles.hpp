@@ -579,27 +579,13 @@ __device__ inline void bin_count_flush(const int* s_hist, int wbase, int* __rest
     }
 }
 // after a barrier: claim each window tile's slots from the counters, which
-// run down to 0 -- the block's entries of tile wbase + k take list places
-// [s_hist[k], s_hist[k] + count) on return.  A thread's tiles are claimed
-// together (each claim waits for its counter, ~1 us), and the lists' starts are
-// added here, a coalesced read, rather than gathered per entry (fill pass of 256
-// uneven frames 43.6 -> 32.4 us, of 64 like frames 17.6 -> 16.5; 1,000,000
-// Gaussian emitters on one frame 33 us both ways: its scattered writes).
-__device__ inline void bin_claim(int* s_hist, int wbase, const int* __restrict__ tile_begin,
-                                 int* __restrict__ tile_left, int cs) {
-    constexpr int PER = BIN_WIN / BIN_THREADS;
-    static_assert(PER * BIN_THREADS == BIN_WIN, "BIN_THREADS threads hold the window");
-    int c[PER], at[PER];
-#pragma unroll
-    for (int j = 0; j < PER; ++j) c[j] = s_hist[j * BIN_THREADS + threadIdx.x];
-#pragma unroll
-    for (int j = 0; j < PER; ++j) {
-        const int tile = wbase + j * BIN_THREADS + (int)threadIdx.x;
-        at[j] = 0;
-        if (c[j]) at[j] = tile_begin[tile] + atomicSub(&tile_left[(size_t)tile * cs], c[j]) - c[j];
+// run down to 0 -- the block's entries of tile wbase + k take [s_hist[k],
+// s_hist[k] + count) on return
+__device__ inline void bin_claim(int* s_hist, int wbase, int* __restrict__ tile_left, int cs) {
+    for (int k = threadIdx.x; k < BIN_WIN; k += blockDim.x) {
+        const int c = s_hist[k];
+        if (c) s_hist[k] = atomicSub(&tile_left[(size_t)(wbase + k) * cs], c) - c;
     }
-#pragma unroll
-    for (int j = 0; j < PER; ++j) s_hist[j * BIN_THREADS + threadIdx.x] = at[j];
 }
 
 __device__ inline void lds_add(double* p, double v) {
