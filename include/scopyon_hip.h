@@ -192,10 +192,10 @@ int smx_splat_accumulate(int n, const double* u, const double* v, const double* 
  * (another is correct, only slower).  Not with a detector epilogue. */
 #define SMX_K_PLACES 3
 /* Or-ed into the tile side: this workspace was binned before by a call with
- * the same FOV layout, tile side, emitter count and list capacity, so its
- * tile counters are back at zero (the fill counts them down) and its tile ->
- * FOV map is current; the binning then skips their initialisation (one
- * launch).  Only with fewer than 65,536 tiles (the one-workgroup counter
+ * the same FOV layout, tile side, emitter count and list capacity (whatever
+ * its tables and quadrant), so its tile counters are back at zero (the fill
+ * counts them down) and its tile -> FOV map is current; the binning then
+ * skips their initialisation (one launch).  Only with fewer than 65,536 tiles (the one-workgroup counter
  * scan); ignored otherwise.  No reference counterpart. */
 #define SMX_TILE_WARM 0x200
 int smx_splat_expected_ts(int n, const double* u, const double* v, const double* w,

@@ -1639,7 +1639,7 @@ static int splat_run(int n, const double* u, const double* v, const double* w, c
         k_format = 1;
     }
     const smx::PhaseFold PF = smx::make_phase_fold(ntab, sat_period > 0 ? sat_period : 1);
-    const bool q32 = (tile_side & SMX_TILE_Q32) != 0;
+    bool q32 = (tile_side & SMX_TILE_Q32) != 0;
     const bool warm = (tile_side & SMX_TILE_WARM) != 0;
     const int side = tile_side & ~(SMX_TILE_Q32 | SMX_TILE_WARM);
     const int lts = side == 16 ? 4 : side == 32 ? 5 : side == 64 ? 6 : -1;
@@ -1673,13 +1673,18 @@ static int splat_run(int n, const double* u, const double* v, const double* w, c
     // about two tiles per emitter at these footprints
     const int cs = smx::agg_count_stride(2LL * n, n_tiles);
 
-    // small launches: the tile pass lists its emitters itself (the 16 and 32
-    // pixel tiles of 16 x 16 quadrants).  The capacity must hold every entry
-    // either way, so that a list too small for the binning is still refused.
+    // small launches: the tile pass lists its emitters itself (16 and 32 pixel
+    // tiles).  The capacity must hold every entry either way, so that a list
+    // too small for the binning is still refused.  Whether lists are made must
+    // not depend on the quadrant: a workspace binned with one may be
+    // accumulated with the other.  So such a launch runs 16 x 16 quadrants
+    // (same bits) whichever were asked for: few emitters leave the one wave of
+    // a 32 x 32 quadrant nothing to gain.
     const long long per_axis = side > 0 ? (m + side - 2) / side + 1 : 0;
-    const bool scan = K && !q32 && lts <= 5 && n > 0 && n <= SCAN_N &&
+    const bool scan = K && lts <= 5 && n > 0 && n <= SCAN_N &&
                       (long long)n * n_tiles <= (lts == 4 ? SCAN_TESTS_16 : SCAN_TESTS) &&
                       list_capacity >= (long long)n * per_axis * per_axis;
+    if (scan) q32 = false;
     smx::HeavyTiles heavy{};
     heavy.cap = K && !scan ? heavy_cap(n_tiles) : 0;
     if (heavy.cap > 0) {
@@ -1689,7 +1694,9 @@ static int splat_run(int n, const double* u, const double* v, const double* w, c
                                              std::max(64LL, HEAVY_TIMES * (list_capacity / n_tiles)));
     }
     if ((stages & 1) && scan) {
-        if (nfov > 1 && !(warm && n_tiles + 1 <= smx::SCAN_MAX)) {
+        // counters and tile map are left as any binning leaves them, for a
+        // warm call that does make lists
+        if (!(warm && n_tiles + 1 <= smx::SCAN_MAX)) {
             hipLaunchKernelGGL(smx::tiles_init_kernel, dim3((n_tiles + 1 + 255) / 256), dim3(256),
                                0, stream, nfov, fovs_dev, n_tiles, ws.tile_count, cs, ws.tile_fov,
                                ws.long_tiles, heavy.list);

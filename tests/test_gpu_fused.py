@@ -202,3 +202,47 @@ def test_heavy_tiles_first(gpu, clustered, spread):
     assert frames[0][0].abs().sum() > 0
     for photons, adc in frames[1:]:
         assert torch.equal(photons, frames[0][0]) and torch.equal(adc, frames[0][1])
+
+
+@pytest.mark.parametrize('nfov,n', [(1, 300), (3, 200), (1, 2100)])
+def test_workspace_across_call_forms(gpu, nfov, n):
+    """A workspace binned by a call that lists its emitters itself (few of them)
+    serves the calls that the interface allows on it: warm calls without phase
+    tables or with the other quadrant, and the tile pass with the other quadrant.
+    Same bits as each call on a workspace of its own."""
+    from scopyon_amd import _device, _lib
+    from scopyon_amd.batched import BatchedSimulator
+    q32, warm = 0x100, 0x200
+    sim = BatchedSimulator(_cfg(), [(61 + f, 64 - f) for f in range(nfov)], n, dt=0.033, seed=2,
+                           tile_side=32, table_precision='float64')
+    sim.weights()
+    t = sim.tables
+
+    def fresh():
+        return torch.full_like(sim.ws, 0x55)
+
+    def call(entry, tile, ws, phase=True):
+        out = torch.zeros_like(sim.photons)
+        _lib.call('smx_splat_{}_ts'.format(entry), sim.n, sim.u.data_ptr(), sim.v.data_ptr(),
+                  sim.w.data_ptr(), sim.key.data_ptr(), sim.fov_id.data_ptr(),
+                  sim.fovs_dev.data_ptr(), sim.nfov, sim.n_tiles, t.sat.data_ptr(), t.sat_elems,
+                  len(t.slot_of), t.ntab, t.period, 1e-9, 1e-18, sim.capacity, 0,
+                  _device.ptr(sim.Ktab if phase else None), sim.k_format, t.m, out.data_ptr(),
+                  ws.data_ptr(), ws.numel(), sim.splatter.status.data_ptr(), _device.stream(), tile)
+        return out
+
+    listed, general = call('expected', 32, fresh()), call('expected', 32, fresh(), phase=False)
+    assert listed.abs().sum() > 0
+    torch.testing.assert_close(listed, general, rtol=1e-12, atol=0)
+    for tile in (32, 32 | q32):
+        for then in (32, 32 | q32):
+            ws = fresh()
+            assert torch.equal(call('expected', tile, ws), listed)
+            assert torch.equal(call('accumulate', then, ws), listed)
+            assert torch.equal(call('expected', then | warm, ws), listed)
+            ws = fresh()
+            call('bin', tile, ws)
+            assert torch.equal(call('accumulate', then, ws), listed)
+            assert torch.equal(call('expected', 32 | warm, ws, phase=False), general)
+            assert torch.equal(call('expected', then | warm, ws), listed)
+    assert sim.status() == 0
