@@ -378,7 +378,8 @@ __global__ void __launch_bounds__(64) sat_col_kernel(int ntab, const double* __r
 // Rows per segment: 32, or 8 where a few tables would leave CUs idle: one
 // table is 250 blocks of 8 rows (sat_rows_kernel 25 us; 16 rows 44, 32 rows
 // 82), and 64 tables are best at 32 (588 us; 620 at 64 rows).
-int sat_segment_rows(int nz) { return nz <= 4 ? 8 : 32; }
+constexpr int kSatFew = 4;
+int sat_segment_rows(int nz) { return nz <= kSatFew ? 8 : 32; }
 
 template <int ZB, bool STAGED>
 int sat_build(const double* radial, int nz, int nr, double res, int ntab, smx::SatLayout L,
@@ -462,8 +463,13 @@ size_t smx_psf_sat_workspace_bytes(int nr, int nz) {
     if (nr < 2 || nz < 0) return 0;
     size_t ntab = 2 * (size_t)nr - 1;
     if (ntab <= (size_t)kSatMax) {
-        const int rows = sat_segment_rows(nz);
-        return (ntab + rows - 1) / rows * ntab * (size_t)nz * sizeof(double);
+        // segment sums; a workspace for nz tables also holds any fewer, whose
+        // segments are shorter
+        auto sums = [&](int tables) {
+            const int rows = sat_segment_rows(tables);
+            return (ntab + rows - 1) / rows * (size_t)tables;
+        };
+        return std::max(sums(nz), sums(std::min(nz, kSatFew))) * ntab * sizeof(double);
     }
     return ntab * (ntab + 1) * (size_t)nz * sizeof(double);
 }

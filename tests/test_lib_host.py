@@ -174,3 +174,17 @@ def test_sorted_tables_limits():
     places = numpy.empty(8, dtype=numpy.int32)
     for nr, ratio in ((4, 1.0), (4, float('nan')), (1, 2.5), (5000, 2.5)):
         assert lib.smx_sat_sorted_places(nr, ratio, places.ctypes.data) == _lib.SMX_EVALUE
+
+
+@pytest.mark.parametrize('nr', [2, 65, 1000, 2048, 2049])
+def test_sat_workspace_holds_any_fewer_tables(nr):
+    """A workspace sized for nz tables serves a build of any fewer: up to four
+    tables are built from segments of 8 rows instead of 32, whose sums are more."""
+    lib = _lib.lib()
+    sizes = [int(lib.smx_psf_sat_workspace_bytes(nr, nz)) for nz in range(70)]
+    assert sizes == sorted(sizes)
+    ntab = 2 * nr - 1
+    if ntab <= 4096:
+        for nz, size in enumerate(sizes):
+            rows = 8 if nz <= 4 else 32
+            assert size >= -(-ntab // rows) * ntab * nz * 8
