@@ -375,16 +375,17 @@ __global__ void __launch_bounds__(64) sat_col_kernel(int ntab, const double* __r
     }
 }
 
-// Rows per segment: 32, or 8 where a few tables would leave CUs idle: one
-// table is 250 blocks of 8 rows (sat_rows_kernel 25 us; 16 rows 44, 32 rows
-// 82), and 64 tables are best at 32 (588 us; 620 at 64 rows).
-constexpr int kSatFew = 4;
-int sat_segment_rows(int nz) { return nz <= kSatFew ? 8 : 32; }
+// Rows per segment.  One height for any number of tables: it sets the order in
+// which a column is added up, and a table's bits must not depend on what else is
+// built with it.  Whole build in us with 8 / 16 / 32 rows: 64 tables 830 / 750 /
+// 735, 53 tables 720 / 670 / 715; one table 52 / 66, of it the row kernel's 250 /
+// 125 / 63 blocks 25 / 44 / 82.
+constexpr int kSegRows = 16;
 
 template <int ZB, bool STAGED>
 int sat_build(const double* radial, int nz, int nr, double res, int ntab, smx::SatLayout L,
               const int* places, size_t stride, double* sums, double* sat, hipStream_t stream) {
-    const int seg = sat_segment_rows(nz), nseg = (ntab + seg - 1) / seg, nzb = (nz + ZB - 1) / ZB;
+    const int seg = kSegRows, nseg = (ntab + seg - 1) / seg, nzb = (nz + ZB - 1) / ZB;
     const size_t lds = sizeof(double2) * ZB * (size_t)nr;
     // every block computes the slopes of its profiles, so a block takes whole
     // rows (64 tables: 168 us, 270 us in panels) unless that leaves CUs idle
@@ -462,15 +463,8 @@ size_t smx_psf_sat_elems(int nr, int period) {
 size_t smx_psf_sat_workspace_bytes(int nr, int nz) {
     if (nr < 2 || nz < 0) return 0;
     size_t ntab = 2 * (size_t)nr - 1;
-    if (ntab <= (size_t)kSatMax) {
-        // segment sums; a workspace for nz tables also holds any fewer, whose
-        // segments are shorter
-        auto sums = [&](int tables) {
-            const int rows = sat_segment_rows(tables);
-            return (ntab + rows - 1) / rows * (size_t)tables;
-        };
-        return std::max(sums(nz), sums(std::min(nz, kSatFew))) * ntab * sizeof(double);
-    }
+    if (ntab <= (size_t)kSatMax)   // segment sums
+        return (ntab + kSegRows - 1) / kSegRows * ntab * (size_t)nz * sizeof(double);
     return ntab * (ntab + 1) * (size_t)nz * sizeof(double);
 }
 

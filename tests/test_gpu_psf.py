@@ -86,3 +86,62 @@ def test_sat_build_sizes(gpu, nr, nz, period):
         ref[1:, 1:] = table.cumsum(axis=0).cumsum(axis=1)
         got = sat[z].cpu().numpy()[rows[:, None] + place[None, :]]
         numpy.testing.assert_allclose(got, ref, rtol=2e-12, atol=0)
+
+
+@pytest.mark.parametrize('nr', [33, 1000])
+@pytest.mark.parametrize('layout', ['plain', 'sorted'])
+def test_sat_bits_do_not_depend_on_the_batch(gpu, nr, layout):
+    """A depth's table built alone and among any others is the same bits."""
+    from scopyon_amd import _device, _lib
+    lib = _lib.lib()
+    rng = numpy.random.RandomState(nr)
+    nz = 67
+    prof = _device.upload(rng.uniform(0.1, 1.0, (nz, nr)), device=gpu)
+    if layout == 'plain':
+        elems = int(lib.smx_psf_sat_elems(nr, 1))
+    else:
+        elems = int(lib.smx_psf_sat_sorted_elems(nr))
+        places = numpy.empty(2 * nr, dtype=numpy.int32)
+        _lib.call('smx_sat_sorted_places', nr, 6.639, places.ctypes.data)
+        places = _device.upload(places, dtype=torch.int32, device=gpu)
+
+    def build(first, count):
+        ws = torch.empty(int(lib.smx_psf_sat_workspace_bytes(nr, count)), dtype=torch.uint8,
+                         device=gpu)
+        sat = torch.empty((count, elems), dtype=torch.float64, device=gpu)
+        args = (prof[first].data_ptr(), count, nr, 1e-9)
+        if layout == 'plain':
+            _lib.call('smx_psf_sat_build', *args, 1, ws.data_ptr(), sat.data_ptr(),
+                      _device.stream())
+        else:
+            _lib.call('smx_psf_sat_build_sorted', *args, places.data_ptr(), ws.data_ptr(),
+                      sat.data_ptr(), _device.stream())
+        return sat
+
+    alone = torch.cat([build(z, 1) for z in range(nz)])
+    assert alone.isfinite().all() and alone.any(dim=1).all()
+    for count in (2, 4, 5, 16, 66, 67):
+        assert torch.equal(build(0, count), alone[:count])
+
+
+def test_tables_do_not_depend_on_how_they_were_asked_for(gpu):
+    """Depth keys met one after another, and in one call: the same tables, also
+    in the copy in the plain layout."""
+    from scopyon_amd import _lib
+    from scopyon_amd._psf import PSFTables
+    keys = [0, 3, 250, 17, 40, 41, 999, -1]
+    kw = dict(pixel_length=16e-6 / 241.0, device=gpu)
+    one = PSFTables('Alexa 647', 6.6e-7, 4.0e-7, 1.0e-6, **kw)
+    for k in keys:
+        one.ensure(numpy.array([k]))
+    all_ = PSFTables('Alexa 647', 6.6e-7, 4.0e-7, 1.0e-6, **kw)
+    all_.ensure(numpy.array(keys))
+    assert one.places is not None and set(one.slot_of) == set(all_.slot_of)
+    lib, side = _lib.lib(), one.ntab + 1     # the plain layout has places without a corner
+    rows = torch.tensor([lib.smx_sat_index_host(side, one.period, a, 0) for a in range(side)])
+    cols = torch.tensor([lib.smx_sat_index_host(side, one.period, 0, b) for b in range(side)])
+    corners = (rows[:, None] + cols).to(gpu)
+    for k in one.slot_of:
+        a, b = one.slot_of[k], all_.slot_of[k]
+        assert torch.equal(one._sat[a], all_._sat[b])
+        assert torch.equal(one.sat[a][corners], all_.sat[b][corners])
