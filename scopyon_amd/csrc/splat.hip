@@ -302,16 +302,17 @@ constexpr int SCORN = (SEDGES * SEDGES + 63) / 64;   // corner loads of a whole 
 
 // Corner a of one axis as a table place, as byte offsets: `main` along a row's
 // run (columns) or of the row (rows); `side` of the row in the side vectors.
-// WIDE: tables of 4 GB and more, offsets in elements (never sorted).
+// WIDE: tables of 4 GB and more (never sorted): the places themselves, which the
+// loads join to a 64-bit offset.
 template <bool WIDE>
 struct SatPlaces {
-    static constexpr unsigned UNIT = WIDE ? 1 : 8;
     const int* places;
     smx::SatLayout L;
     int ntab;
     __device__ int2 row(int a) const {
-        if (WIDE || !places) {
-            const int r = (int)((unsigned)L.row_part(a) * UNIT);
+        if (WIDE) return make_int2(L.place(a), 0);
+        if (!places) {
+            const int r = (int)((unsigned)L.row_part(a) * 8);
             return make_int2(r, r);
         }
         const int p = places[a];
@@ -319,7 +320,8 @@ struct SatPlaces {
     }
     // bit 0: the offset goes with the row's `side` instead of its `main`
     __device__ int col(int b) const {
-        if (WIDE || !places) return (int)((unsigned)L.col_part(b) * UNIT);
+        if (WIDE) return L.place(b);
+        if (!places) return (int)((unsigned)L.col_part(b) * 8);
         const int side = ntab + 1;
         if (b == 0) return (side * side * 8) | 1;
         if (b == ntab) return ((side + 1) * side * 8) | 1;
@@ -357,7 +359,7 @@ __device__ inline void load_corners(const TileArgs& A, const SatWaveLds& wl, int
         const int2 r = rows[row];
         const int col = cols[idx - __mul24(row, W1)];
         if (WIDE)
-            out[q] = smx::gload((const double*)T + ((unsigned)r.x + (unsigned)col));
+            out[q] = smx::gload((const double*)T + ((size_t)r.x * A.L.width + col));
         else
             out[q] = smx::gload((const double*)(T + ((unsigned)(col & 1 ? r.y : r.x) +
                                                      (unsigned)(col & ~1))));

@@ -130,3 +130,66 @@ def test_sorted_tables_equal_plain_layout(gpu, mag, shape, n, spread):
                   *t.splat_tables()[2:], t.m, None, ws.data_ptr(), ws.numel(),
                   sim.splatter.status.data_ptr(), _device.stream(), None, None, sim.det, 0, 0, 0,
                   None, None, got.data_ptr(), 0, 32)
+
+
+@pytest.mark.parametrize('nr', [11600, 33000])
+def test_splat_from_wide_tables(gpu, nr):
+    """Tables of more than 2^29 corners (4 GB) and of more than 2^32, whose
+    offsets need 64 bits: 23 and 66 um across on 66.4 cells a pixel.  Corner
+    (a, b) holds f(a) f(b) with whole f, so every pixel integral is an exact whole
+    number, and the frame lies at the table's last corner or its first."""
+    from scopyon_amd import _device, _epifm, _lib
+    side, ntab = 2 * nr, 2 * nr - 1
+    pl, shape = 66.39e-9, (40, 33)
+    period = 66
+    lib = _lib.lib()
+    f = numpy.arange(side) + numpy.arange(side) % 7
+    place = numpy.arange(side) % period * (-(-side // period)) + numpy.arange(side) // period
+    for a in (0, 1, 65, 66, side - 1):
+        assert lib.smx_sat_index_host(side, period, 0, a) == place[a]
+    width = period * -(-side // period)
+    assert int(lib.smx_psf_sat_elems(nr, period)) == width * width
+    axis = numpy.zeros(width)
+    axis[place] = f
+    axis = torch.as_tensor(axis, device=gpu)
+    table = torch.empty((width, width), dtype=torch.float64, device=gpu)
+    for rows in range(0, width, 1024):
+        torch.outer(axis[rows:rows + 1024], axis, out=table[rows:rows + 1024])
+    geom = _epifm.FrameGeometry(*shape, pl, 0.0, 0.0)
+    fovs = torch.from_numpy(numpy.frombuffer(bytes(geom.fov), dtype=numpy.uint8).copy()).to(gpu)
+    half, res = 1e-9 * (ntab - 1) * 0.5, 1e-9
+    # centres that put the frame at the end of the footprint, at its start, and
+    # once across its last corner
+    at = numpy.array([[-half + 15 * pl, -half + 12 * pl], [half - 14.3 * pl, half - 11.6 * pl],
+                      [-half + 1.7 * pl, half - 3.2 * pl]])
+    n = len(at)
+    u, v = (_device.upload(at[:, k], device=gpu) for k in (0, 1))
+    w = torch.tensor([1.0, 2.0, 4.0], dtype=torch.float64, device=gpu)
+    key = torch.zeros(n, dtype=torch.int32, device=gpu)
+    cap = n * geom.n_tiles
+    ws = torch.empty(lib.smx_splat_workspace_bytes(n, geom.n_tiles, cap), dtype=torch.uint8,
+                     device=gpu)
+    status = torch.zeros(1, dtype=torch.int32, device=gpu)
+    out = torch.empty(shape, dtype=torch.float64, device=gpu)
+    _lib.call('smx_splat_expected', n, u.data_ptr(), v.data_ptr(), w.data_ptr(), key.data_ptr(),
+              None, fovs.data_ptr(), 1, geom.n_tiles, table.data_ptr(), table.numel(), 1, ntab,
+              period, res, 1.0, cap, 0, None, 0, 0, out.data_ptr(), ws.data_ptr(), ws.numel(),
+              status.data_ptr(), _device.stream())
+    got = out.cpu().numpy()
+    del table
+    torch.cuda.empty_cache()
+    assert int(status.item()) == 0
+    want = numpy.zeros(shape)
+    for (x, y), weight in zip(at, (1.0, 2.0, 4.0)):
+        sums = []
+        for c, size in ((x, shape[0]), (y, shape[1])):
+            o = size * pl * 0.5 + c - half
+            # the footprint's pixels, and its table cells cut at their edges
+            # (_epifm.py:241-263)
+            k = numpy.arange(size)
+            inside = (k >= numpy.floor(o / pl)) & (k < numpy.ceil((size * pl * 0.5 + c + half) / pl))
+            edge = numpy.ceil((numpy.arange(size + 1) * pl - o) / res)
+            sums.append(inside * numpy.diff(f[numpy.clip(edge, 0, ntab).astype(int)]))
+        want += weight * numpy.outer(*sums)
+    assert (want > 0).mean() > 0.5
+    assert numpy.array_equal(got, want)
