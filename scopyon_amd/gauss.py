@@ -282,9 +282,9 @@ class _NLL(torch.autograd.Function):
     def backward(ctx, g_loss):
         (grad,) = ctx.saved_tensors
         model = ctx.model
-        if (torch.is_grad_enabled() and g_loss.requires_grad) or not _has_storage(g_loss):
-            # create_graph (the product stays differentiable in g_loss) and
-            # batched gradients (vmap): plain tensor operations
+        if (torch.is_grad_enabled() and g_loss.requires_grad) or not _readable(g_loss):
+            # create_graph (the product stays differentiable in g_loss), forward
+            # mode and batched gradients (vmap): plain tensor operations
             scale = torch.repeat_interleave(
                 g_loss.to(torch.float32),
                 torch.as_tensor(numpy.diff(model.pix_offsets), device=grad.device))
@@ -292,13 +292,14 @@ class _NLL(torch.autograd.Function):
         return None, model.scale_frames(grad, g_loss), None
 
 
-def _has_storage(t):
-    """False for the wrapper tensors of vmap and the like, which no kernel can read."""
+def _readable(t):
+    """Whether a kernel that reads t by its address sees all of it: not the
+    wrapper tensors of vmap and the like, no forward-mode tangent, no pending sign."""
     try:
         t.data_ptr()
     except RuntimeError:
         return False
-    return True
+    return not t.is_neg() and torch.autograd.forward_ad.unpack_dual(t).tangent is None
 
 
 def render(model, x, y, z, I, sigma=None, frame_id=None):

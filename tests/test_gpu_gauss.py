@@ -496,3 +496,31 @@ def test_nll_gradient_scaling(gpu, shapes):
         a = sum(sizes[:f])
         assert torch.equal(gb[f, a:a + sizes[f]], base[a:a + sizes[f]])
         assert gb[f].count_nonzero() == base[a:a + sizes[f]].count_nonzero()
+
+
+def test_nll_gradient_in_forward_mode(gpu):
+    """Upstream gradients with a tangent, or with a pending sign: the image
+    gradient carries the tangent and the sign, as the tensor product does."""
+    import torch.autograd.forward_ad as fw
+    from scopyon_amd.gauss import poisson_nll
+    rng = numpy.random.RandomState(3)
+    shapes = [(20, 31), (7, 9)]
+    sizes = [a * b for a, b in shapes]
+    m = _model(shapes)
+    k = _dev(rng.poisson(20.0, sum(sizes)))
+    mu = _dev(rng.uniform(1.0, 40.0, sum(sizes))).requires_grad_()
+    w, t = (torch.as_tensor(rng.uniform(-2.0, 2.0, 2), device='cuda') for _ in range(2))
+
+    def scaled(weight):
+        base = torch.empty_like(mu)
+        m.nll(mu.detach(), k, base)
+        return torch.cat([b * f for b, f in zip(base.split(sizes), weight.float())])
+
+    with fw.dual_level():
+        (g,) = torch.autograd.grad(poisson_nll(m, mu, k), mu, fw.make_dual(w, t))
+        primal, tangent = fw.unpack_dual(g)
+        assert torch.equal(primal, scaled(w)) and torch.equal(tangent, scaled(t))
+    lazy = torch.complex(t, w).conj().imag
+    assert lazy.is_neg()
+    (g,) = torch.autograd.grad(poisson_nll(m, mu, k), mu, lazy)
+    assert torch.equal(g, scaled(-w))
