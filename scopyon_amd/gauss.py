@@ -183,9 +183,19 @@ class GaussianModel:
                   _device.stream())
         return self.loss
 
+    def holds_pixels(self, t):
+        """Whether t is an image of all frames as the kernels read it."""
+        return (t.shape == (self.n_pix,) and t.dtype == torch.float32 and t.is_cuda and
+                t.is_contiguous())
+
     def scale_frames(self, grad_mu, weight):
         """grad_mu with every frame's pixels times that frame's weight (float64
         device tensor, one per frame): dL/dmu of a weighted sum of losses."""
+        if not self.holds_pixels(grad_mu):
+            raise TypeError('grad_mu must be a contiguous float32 CUDA tensor of all {} pixels'
+                            .format(self.n_pix))
+        if weight.shape != (self.nframes,) or not weight.is_cuda:
+            raise TypeError('weight must be a CUDA tensor with one entry per frame')
         weight = weight.detach().to(torch.float64).contiguous()
         out = torch.empty_like(grad_mu)
         _lib.call('smx_gauss_scale_frames', grad_mu.data_ptr(), weight.data_ptr(),
@@ -282,9 +292,12 @@ class _NLL(torch.autograd.Function):
     def backward(ctx, g_loss):
         (grad,) = ctx.saved_tensors
         model = ctx.model
-        if (torch.is_grad_enabled() and g_loss.requires_grad) or not _readable(g_loss):
+        if ((torch.is_grad_enabled() and g_loss.requires_grad) or not _readable(g_loss) or
+                not model.holds_pixels(grad) or not _readable(grad)):
             # create_graph (the product stays differentiable in g_loss), forward
-            # mode and batched gradients (vmap): plain tensor operations
+            # mode, batched gradients (vmap), and an image of another shape,
+            # stride or type (mu's, or a saved-tensor hook's): plain tensor
+            # operations, which refuse what does not fit
             scale = torch.repeat_interleave(
                 g_loss.to(torch.float32),
                 torch.as_tensor(numpy.diff(model.pix_offsets), device=grad.device))

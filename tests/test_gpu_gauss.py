@@ -524,3 +524,37 @@ def test_nll_gradient_in_forward_mode(gpu):
     assert lazy.is_neg()
     (g,) = torch.autograd.grad(poisson_nll(m, mu, k), mu, lazy)
     assert torch.equal(g, scaled(-w))
+
+
+def test_nll_gradient_of_other_image_layouts(gpu):
+    """The backward's kernel reads an image of all pixels in order.  A transposed
+    image is refused as by the tensor product, never returned transposed; one row
+    of pixels, strided pixels and a saved-tensor hook's other type give the
+    gradient of the plain image."""
+    from scopyon_amd.gauss import poisson_nll
+    rng = numpy.random.RandomState(8)
+    m = _model([(24, 24)])
+    k = _dev(rng.poisson(20.0, 576))
+    pixels = _dev(rng.uniform(1.0, 40.0, 576))
+    base = torch.empty_like(pixels)
+    m.nll(pixels, k, base)
+
+    def gradient(mu):
+        (g,) = torch.autograd.grad(poisson_nll(m, mu, k).sum(), mu)
+        assert g.shape == mu.shape
+        return g.reshape(-1)
+
+    assert torch.equal(gradient(pixels.clone().requires_grad_()), base)
+    assert torch.equal(gradient(pixels.reshape(1, -1).requires_grad_()), base)
+    strided = torch.stack([pixels, pixels], 1)[:, 0].requires_grad_()
+    assert not strided.is_contiguous() and torch.equal(gradient(strided), base)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.double(), lambda t: t):
+        mu = pixels.clone().requires_grad_()
+        assert torch.equal(gradient(mu), base)
+    for mu in (pixels.reshape(24, 24).t().requires_grad_(), pixels.reshape(24, 24).requires_grad_()):
+        with pytest.raises(RuntimeError):
+            gradient(mu)
+    with pytest.raises(TypeError):
+        m.scale_frames(base[:-1], torch.ones(1, dtype=torch.float64, device='cuda'))
+    with pytest.raises(TypeError):
+        m.scale_frames(base, torch.ones(2, dtype=torch.float64, device='cuda'))
