@@ -23,19 +23,29 @@ def ptr(t):
     return None if t is None else t.data_ptr()
 
 
+def upload(a, dtype=torch.float64, device=None):
+    """Device copy of a host array, complete on return: for what an object keeps,
+    which may be used on other streams than the one it was made on."""
+    device = device or require_gpu()
+    return torch.from_numpy(numpy.ascontiguousarray(a)).to(device=device, dtype=dtype,
+                                                           non_blocking=False)
+
+
 UPLOAD_STAGED = 1 << 18   # bytes
 
 
-def upload(a, dtype=torch.float64, device=None):
+def stage(a, dtype=torch.float64, device=None):
+    """Device copy of a host array, ordered on the current stream: for what only the
+    work that the caller queues on this stream reads.  Small arrays go through
+    pinned memory: a copy from pageable memory would wait for the kernels before
+    it on the stream (torch keeps the pinned block until it is read)."""
     device = device or require_gpu()
     a = numpy.ascontiguousarray(a)
-    if 0 < a.nbytes <= UPLOAD_STAGED:
-        # through pinned memory: a copy from pageable memory would wait for the
-        # kernels before it on the stream (torch keeps the block until it is read)
-        src = torch.from_numpy(a)
-        staged = torch.empty(src.shape, dtype=dtype, pin_memory=True)
-        return staged.copy_(src).to(device=device, non_blocking=True)
-    return torch.from_numpy(a).to(device=device, dtype=dtype, non_blocking=False)
+    if not 0 < a.nbytes <= UPLOAD_STAGED:
+        return upload(a, dtype, device)
+    src = torch.from_numpy(a)
+    staged = torch.empty(src.shape, dtype=dtype, pin_memory=True)
+    return staged.copy_(src).to(device=device, non_blocking=True)
 
 
 class Arena:

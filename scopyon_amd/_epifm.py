@@ -369,10 +369,10 @@ class _EPIFMSimulator:
             if count:      # one vector draw gives the values of as many single ones
                 vals[drawn] = (rng.host_exponentials(beta, count) if isinstance(rng, PhiloxRNG)
                                else rng.exponential(scale=beta, size=count)) * N_emit0
-            idx = _device.upload(numpy.array([s for s, _ in new]), dtype=torch.int64,
-                                 device=self.device)
-            self._budget[idx] = _device.upload(vals, device=self.device)
-        self._slots = _device.upload(slots, dtype=torch.int32, device=self.device)
+            idx = _device.stage(numpy.array([s for s, _ in new]), dtype=torch.int64,
+                                device=self.device)
+            self._budget[idx] = _device.stage(vals, device=self.device)
+        self._slots = _device.stage(slots, dtype=torch.int32, device=self.device)
         self._slot_ids = m_ids
         return self._slots
 
@@ -391,7 +391,7 @@ class _EPIFMSimulator:
             raise TypeError(c.filter_error)
         keys = depth_keys(p[:, 0], c.detector_focal_point[0], c.depth_cutoff)
         self.tables.ensure(keys)
-        dev = _device.upload(p, device=self.device)
+        dev = _device.stage(p, device=self.device)
         depth, u, v = dev[:, 0].contiguous(), dev[:, 1].contiguous(), dev[:, 2].contiguous()
         p_state = dev[:, 4].contiguous()
         budget = slots = None
@@ -399,7 +399,7 @@ class _EPIFMSimulator:
             slots = self._bleach_slots(_molecule_ids(p[:, 3]), states, rng)
             budget = self._budget
         w, key, ps = self.splatter.weights(depth, p_state, unit_time, budget, slots,
-                                           self.tables.slot_map())
+                                           self.tables.slot_map(_device.stage))
         self.splatter.splat(u, v, w, key, self.fovs_dev, 1, self.geom.n_tiles, camera)
         if full_output:
             pending.append((p, unit_time, w, ps))
@@ -455,9 +455,9 @@ class _EPIFMSimulator:
         count = int((uidx[-1] + flag[-1]).item())
         _status_check(self.splatter.status)
         if noise is not None:
-            noise = _device.upload(noise, device=self.device)
-        uni = _device.upload(rng.random_sample(count) if count else numpy.zeros(1),
-                             device=self.device)
+            noise = _device.stage(noise, device=self.device)
+        uni = _device.stage(rng.random_sample(count) if count else numpy.zeros(1),
+                            device=self.device)
         E_common = float(c.detector_qeff * ((0.0 + c.background_mean) if c.background_switch
                                             else 0.0))
         T_common = _device.ARENA.typed('det_tcommon', int(_lib.lib().smx_emccd_common_elems()),
@@ -505,14 +505,14 @@ class _EPIFMSimulator:
         # reference order: the noise (CMOS: one RandomState.choice uniform per
         # pixel; CCD: one vector normal draw), then rng.poisson per pixel
         if cmos:
-            noise = _device.upload(rng.random_sample(n), device=self.device)
+            noise = _device.stage(rng.random_sample(n), device=self.device)
         elif c.detector_readout_noise > 0:
-            noise = _device.upload(rng.normal(0, c.detector_readout_noise, shape),
-                                   device=self.device)
+            noise = _device.stage(rng.normal(0, c.detector_readout_noise, shape),
+                                  device=self.device)
         else:
             noise = None
         signal = rng.poisson(E.cpu().numpy().reshape(shape)).astype(numpy.float64)
-        sig = _device.upload(signal, device=self.device)
+        sig = _device.stage(signal, device=self.device)
         _lib.call('smx_adc_parity', n, sig.data_ptr(), _device.ptr(noise), _device.ptr(tv),
                   _device.ptr(tc), tn, _device.ptr(gain_map), _device.ptr(offset_map), self.det,
                   adc.data_ptr(), st)

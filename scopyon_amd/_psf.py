@@ -126,8 +126,8 @@ class PSFTables:
             _lib.call('smx_psf_radial_gaussian', self.nr, RES, self.radial_width,
                       radial.data_ptr(), _device.stream())
         else:
-            depths = _device.upload(numpy.array([self._depth_of(k) for k in keys]),
-                                    device=self.device)
+            depths = _device.stage(numpy.array([self._depth_of(k) for k in keys]),
+                                   device=self.device)
             j0w = _device.ARENA.typed('psf_j0', self.nr * 100, torch.float64, self.device)
             _lib.call('smx_psf_radial_born_wolf', depths.data_ptr(), nz, self.nr, RES, self.alpha,
                       self.gamma, self.scale, j0w.data_ptr(), radial.data_ptr(), _device.stream())
@@ -212,14 +212,15 @@ class PSFTables:
                       self.m, self._Kfold.data_ptr(), _device.stream())
         return self._Kfold
 
-    def slot_map(self):
-        """Device int32 table: key index -> slot (-1 if not built)."""
+    def slot_map(self, copy=_device.upload):
+        """Device int32 table: key index -> slot (-1 if not built); `copy`:
+        _device.upload, or _device.stage for one use on the current stream."""
         m = numpy.full(self.n_keys, -1, dtype=numpy.int32)
         for k, s in self.slot_of.items():
             m[self.key_index(k)] = s
         if self.gaussian:
             m[:] = self.slot_of.get(0, -1)
-        return _device.upload(m, dtype=torch.int32, device=self.device)
+        return copy(m, dtype=torch.int32, device=self.device)
 
     def prebuild_all(self):
         """Build every depth key (0 .. cutoff) plus the cutoff key."""
@@ -286,7 +287,7 @@ class LUTTables:
         else:
             k = 2.0 * numpy.pi / wavelength
             alpha, gamma = k * na, k * numpy.power(na / 2, 2)
-            depths = _device.upload(self.slice_depths, device=self.device)
+            depths = _device.stage(self.slice_depths, device=self.device)
             j0w = torch.empty(self.nb * 100, dtype=torch.float64, device=self.device)
             _lib.call('smx_psf_radial_born_wolf', depths.data_ptr(), self.nz, self.nb, dr, alpha,
                       gamma, alpha * alpha / numpy.pi, j0w.data_ptr(), self.radial.data_ptr(), st)

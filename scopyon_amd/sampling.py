@@ -96,14 +96,14 @@ def trajectory_predrawn(x0, scale, xi, boundary=0, lower=None, upper=None, state
     nstates = scale.shape[1] if T else (1 if pacc is None else pacc.shape[1])
     xs = torch.empty((T + 1, n, ndim), dtype=torch.float64, device=dev)
     states = torch.empty((T + 1, n), dtype=torch.int32, device=dev)
-    d_x0 = _device.upload(x0, device=dev)
-    d_scale = _device.upload(scale if T else numpy.zeros((1, nstates, ndim)), device=dev)
-    d_xi = _device.upload(xi if T else numpy.zeros((1, n, ndim)), device=dev)
-    d_s0 = None if state0 is None else _device.upload(state0, dtype=torch.int32, device=dev)
-    d_lo = None if lower is None else _device.upload(lower, device=dev)
-    d_hi = None if upper is None else _device.upload(upper, device=dev)
-    d_pacc = None if pacc is None else _device.upload(pacc, device=dev)
-    d_tu = None if trans_u is None else _device.upload(trans_u, device=dev)
+    d_x0 = _device.stage(x0, device=dev)
+    d_scale = _device.stage(scale if T else numpy.zeros((1, nstates, ndim)), device=dev)
+    d_xi = _device.stage(xi if T else numpy.zeros((1, n, ndim)), device=dev)
+    d_s0 = None if state0 is None else _device.stage(state0, dtype=torch.int32, device=dev)
+    d_lo = None if lower is None else _device.stage(lower, device=dev)
+    d_hi = None if upper is None else _device.stage(upper, device=dev)
+    d_pacc = None if pacc is None else _device.stage(pacc, device=dev)
+    d_tu = None if trans_u is None else _device.stage(trans_u, device=dev)
     _lib.call('smx_brownian_predrawn', n, ndim, T, nstates, d_x0.data_ptr(), _device.ptr(d_s0),
               d_scale.data_ptr(), d_xi.data_ptr(), boundary, _device.ptr(d_lo), _device.ptr(d_hi),
               _device.ptr(d_pacc), _device.ptr(d_tu), xs.data_ptr(), states.data_ptr(),
@@ -165,24 +165,24 @@ def _philox_walk(rng, x0, D_tab, moves, boundary=0, lower=None, upper=None, stat
         raise NotImplementedError('PhiloxRNG sampling supports ndim <= 3')
     D_tab = numpy.asarray(D_tab, dtype=float).reshape(-1, ndim)
     nstates = D_tab.shape[0]
-    xs = [_device.upload(x0[:, d].copy(), device=dev) if d < ndim else
+    xs = [_device.stage(x0[:, d].copy(), device=dev) if d < ndim else
           torch.zeros(1, dtype=torch.float64, device=dev) for d in range(3)]
     traj = numpy.empty((len(moves) + 1, n, ndim))
     traj[0] = x0
     s0 = numpy.zeros(n, dtype=numpy.int32) if state0 is None else numpy.asarray(state0, numpy.int32)
     states = numpy.empty((len(moves) + 1, n), dtype=numpy.int32)
     states[0] = s0
-    d_state = _device.upload(s0, dtype=torch.int32, device=dev)
+    d_state = _device.stage(s0, dtype=torch.int32, device=dev)
     lo = _lib.host_doubles(lower[:ndim] if lower is not None else [], 3)
     hi = _lib.host_doubles(upper[:ndim] if upper is not None else [], 3)
-    d_D = _device.upload(numpy.ascontiguousarray(D_tab), device=dev)
+    d_D = _device.stage(numpy.ascontiguousarray(D_tab), device=dev)
     for k, dt in enumerate(moves):
         d_pacc = None
         if transmat is not None:
             P = 1 - numpy.exp(-transmat * dt)
             assert (P.sum(axis=1) <= 1.0).all()
             P.ravel()[::nstates + 1] = 1.0 - P.sum(axis=1)
-            d_pacc = _device.upload(numpy.ascontiguousarray(P.cumsum(axis=1)), device=dev)
+            d_pacc = _device.stage(numpy.ascontiguousarray(P.cumsum(axis=1)), device=dev)
         _lib.call('smx_brownian_philox_states', n, ndim, xs[0].data_ptr(), xs[1].data_ptr(),
                   xs[2].data_ptr(), d_state.data_ptr(), nstates, d_D.data_ptr(), float(dt),
                   boundary, lo, hi, _device.ptr(d_pacc), rng.seed, rng.next_counter(), 0,

@@ -235,3 +235,29 @@ def test_reference_example_images(gpu):
         img, info = scopyon_amd.form_image(part, config=config, rng=rng, full_output=True)
         exact, worst, n_bg = agree(img, info, png[:, :, ch])
         assert n_bg > 100_000 and exact > 0.99 and worst <= 1, (ch, exact, worst, n_bg)
+
+
+def test_uploads_are_complete_for_other_streams(gpu):
+    """What an object keeps on the device is there for work on any stream when the
+    upload returns, however busy the stream it was made on; staged copies are
+    ordered on the caller's stream, in every type, small and large."""
+    import torch
+    from scopyon_amd import _device
+    side = torch.cuda.Stream()
+    a = numpy.random.RandomState(1).uniform(1.0, 2.0, 4000)
+    for _ in range(3):
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(50000000)
+            up = _device.upload(a)
+        seen = up.clone()            # on the default stream
+        torch.cuda.synchronize()
+        assert numpy.array_equal(seen.cpu().numpy(), a)
+        side.synchronize()
+    for n in (0, 1, 4000, 100000):
+        for dtype in (torch.float64, torch.int32, torch.int64):
+            want = (numpy.arange(n) * 1.5).astype(numpy.float64)
+            with torch.cuda.stream(side):
+                torch.cuda._sleep(5000000)
+                twice = _device.stage(want, dtype=dtype, device=gpu) * 2
+                got = twice.cpu()
+            assert torch.equal(got, torch.as_tensor(want).to(dtype) * 2)
