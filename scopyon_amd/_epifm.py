@@ -295,14 +295,28 @@ class Splatter:
                   ws.data_ptr(), ws.numel(), self.status.data_ptr(), _device.stream())
 
 
-def _status_check(status):
-    s = int(status.item())
+def _status_check(status, bits=~0):
+    s = int(status.item()) & bits
     if s & 2:
         raise RuntimeError('scopyon_amd: splat tile list capacity exceeded')
     if s & 8:
         raise RuntimeError('scopyon_amd: a PSF table needed by an emitter was not built')
     if s & 4:
         raise ValueError('probabilities contain NaN')
+
+
+def _rewind(rng):
+    """Function that gives back what is drawn from rng after this call, or None for
+    a generator whose state cannot be put back."""
+    if isinstance(rng, PhiloxRNG):
+        return lambda: None      # counted per frame, nothing is drawn on the host
+    if hasattr(rng, 'get_state') and hasattr(rng, 'set_state'):
+        state = rng.get_state()
+        return lambda: rng.set_state(state)
+    if hasattr(rng, 'bit_generator'):
+        state = rng.bit_generator.state
+        return lambda: setattr(rng.bit_generator, 'state', state)
+    return None
 
 
 def _molecule_ids(column):
@@ -402,9 +416,9 @@ class _EPIFMSimulator:
                                            self.tables.slot_map(_device.stage))
         self.splatter.splat(u, v, w, key, self.fovs_dev, 1, self.geom.n_tiles, camera)
         if full_output:
-            pending.append((p, unit_time, w, ps))
+            pending.append((p, _molecule_ids(p[:, 3]), unit_time, w, ps))
 
-    def _true_data(self, p, unit_time, w, ps, optinfo):
+    def _true_data(self, p, m_ids, unit_time, w, ps, optinfo):
         """Per-molecule sums of _epifm.py:1321-1333."""
         w = w.cpu().numpy()
         ps = ps.cpu().numpy()
@@ -412,14 +426,28 @@ class _EPIFMSimulator:
         u, v = unit_time * p[:, 1], unit_time * p[:, 2]
         rows = 0.0 + numpy.column_stack([numpy.full(len(p), unit_time), unit_time * ps, u, v, u, v,
                                          unit_time * depth, w])
-        for m, row in zip(_molecule_ids(p[:, 3]), rows):
+        for m, row in zip(m_ids, rows):
             if m in optinfo:
                 optinfo[m] += row
             else:
                 optinfo[m] = row.copy()
 
     # ---- detector ----
+    def _check_splat(self, rewind=None):
+        """Raises what the splat reported, the random numbers drawn ahead given back."""
+        try:
+            _status_check(self.splatter.status, 2 | 8)
+        except RuntimeError:
+            if rewind is not None:
+                rewind()
+            raise
+
     def detector(self, camera, rng, full_output):
+        # the splat's status is read only after the first draws (the wait for the GPU
+        # falls behind them): a frame that fails there gives them back
+        rewind = _rewind(rng)
+        if rewind is None:
+            self._check_splat()
         c = self.configs
         n = camera.numel()
         if c.detector_type not in ('EMCCD', 'CCD', 'CMOS'):
@@ -430,7 +458,7 @@ class _EPIFMSimulator:
         adc = torch.empty(n, dtype=torch.float64, device=self.device)
         gain_map, offset_map = (None, None) if self._maps is None else self._maps
         if c.detector_type != 'EMCCD':
-            return self._photon_detector(camera, rng, E, adc, gain_map, offset_map)
+            return self._photon_detector(camera, rng, E, adc, gain_map, offset_map, rewind)
         if isinstance(rng, PhiloxRNG):
             frame = self._philox_frame
             self._philox_frame += 1
@@ -453,7 +481,7 @@ class _EPIFMSimulator:
         noise = (rng.normal(0, c.detector_readout_noise, shape) if c.detector_readout_noise > 0
                  else None)
         count = int((uidx[-1] + flag[-1]).item())
-        _status_check(self.splatter.status)
+        self._check_splat(rewind)
         if noise is not None:
             noise = _device.stage(noise, device=self.device)
         uni = _device.stage(rng.random_sample(count) if count else numpy.zeros(1),
@@ -484,7 +512,7 @@ class _EPIFMSimulator:
                           _device.upload(cdf, device=self.device), len(cdf))
         return self._cmos
 
-    def _photon_detector(self, camera, rng, E, adc, gain_map, offset_map):
+    def _photon_detector(self, camera, rng, E, adc, gain_map, offset_map, rewind):
         """CCD and CMOS (_epifm.py:329-353, 418-433, 1443-1469): Poisson
         photo-electrons plus Gaussian (CCD) or tabulated (CMOS) readout noise."""
         c = self.configs
@@ -511,7 +539,9 @@ class _EPIFMSimulator:
                                   device=self.device)
         else:
             noise = None
-        signal = rng.poisson(E.cpu().numpy().reshape(shape)).astype(numpy.float64)
+        expected = E.cpu().numpy().reshape(shape)
+        self._check_splat(rewind)
+        signal = rng.poisson(expected).astype(numpy.float64)
         sig = _device.stage(signal, device=self.device)
         _lib.call('smx_adc_parity', n, sig.data_ptr(), _device.ptr(noise), _device.ptr(tv),
                   _device.ptr(tc), tn, _device.ptr(gain_map), _device.ptr(offset_map), self.det,
@@ -565,8 +595,13 @@ class _EPIFMSimulator:
                 continue
             self._substep(particles, unit_time, camera, fluorescence_states, rng, pending,
                           full_output)
+        philox_frame = self._philox_frame
         E, adc = self.detector(camera, rng, full_output)
-        _status_check(self.splatter.status)
+        try:
+            _status_check(self.splatter.status)
+        except RuntimeError:      # from the splat: this frame was not formed
+            self._philox_frame = philox_frame
+            raise
         # the weights come to the host only now: the detector's random numbers
         # are drawn while the GPU still forms the image
         optinfo = {}

@@ -261,3 +261,56 @@ def test_uploads_are_complete_for_other_streams(gpu):
                 twice = _device.stage(want, dtype=dtype, device=gpu) * 2
                 got = twice.cpu()
             assert torch.equal(got, torch.as_tensor(want).to(dtype) * 2)
+
+
+@pytest.mark.parametrize('detector', ['EMCCD', 'CCD', 'CMOS'])
+@pytest.mark.parametrize('kind', ['state', 'plain', 'philox'])
+def test_failing_frame_leaves_the_generator(gpu, detector, kind):
+    """A splat that reports an overflow, and a bad molecule id with ground truth,
+    raise with the generator as it was, also one whose state cannot be put back."""
+    import scopyon_amd
+    from scopyon_amd import _epifm
+    ov = {'detector': {'type': detector, 'image_size': [24, 20], 'exposure_time': 0.033},
+          'magnification': 100.0}
+    sim = _epifm._EPIFMSimulator(_epifm.EPIFMConfigs(product_config(ov).default,
+                                                     rng=numpy.random.RandomState(0)))
+    source = numpy.random.RandomState(5)
+
+    class Plain:    # no state to read
+        def __getattr__(self, name):
+            if name in ('normal', 'random_sample', 'poisson', 'standard_normal'):
+                return getattr(source, name)
+            raise AttributeError(name)
+
+    rng = {'state': source, 'plain': Plain(), 'philox': scopyon_amd.PhiloxRNG(5)}[kind]
+    rows = numpy.column_stack([numpy.zeros(9), numpy.linspace(-1e-6, 1e-6, 9), numpy.zeros(9),
+                               numpy.arange(9), numpy.ones(9)])
+
+    def states():
+        return [x.tolist() if hasattr(x, 'tolist') else x for x in source.get_state()]
+
+    good, _ = sim.output_frame([(0.0, rows)], rng=rng)
+    before, frame = states(), sim._philox_frame
+    splat = sim.splatter.splat
+
+    def overflowing(*args, **kwargs):
+        splat(*args, **kwargs)
+        sim.splatter.status |= 2
+
+    sim.splatter.splat = overflowing
+    for full in (False, True):
+        with pytest.raises(RuntimeError, match='capacity'):
+            sim.output_frame([(0.0, rows)], rng=rng, full_output=full)
+        assert states() == before and sim._philox_frame == frame
+    sim.splatter.splat = splat
+    bad = rows.copy()
+    bad[4, 3] = numpy.nan
+    with pytest.raises(ValueError):
+        sim.output_frame([(0.0, bad)], rng=rng, full_output=True)
+    assert states() == before and sim._philox_frame == frame
+    again, _ = sim.output_frame([(0.0, rows)], rng=rng)
+    assert not numpy.array_equal(again[:, :, 1], good[:, :, 1])
+    if kind != 'philox':
+        assert states() != before
+    else:
+        assert sim._philox_frame == frame + 1
