@@ -47,6 +47,13 @@ def layout_period(pixel_length):
     return p if 2 <= p <= 4096 else 1
 
 
+def sat_batch(nr):
+    """Tables built in one call: 64, or 8 where a table's scratch is not a few MB of
+    segment sums but the row sums of every cell (radial cutoffs above 2 um: 134 MB
+    and more)."""
+    return 64 if _lib.lib().smx_psf_sat_workspace_bytes(nr, 1) <= 16 << 20 else 8
+
+
 class PSFTables:
     """Per-depth-key SATs for one fluorophore/PSF model on one device."""
 
@@ -135,8 +142,7 @@ class PSFTables:
 
     def _build(self, radial, out, places):
         """Summed-area tables of the profiles into out (nz, elems)."""
-        # in batches so the scratch stays bounded (~1 MB per table)
-        batch, nz = 64, radial.shape[0]
+        batch, nz = sat_batch(self.nr), radial.shape[0]
         for s in range(0, nz, batch):
             m = min(batch, nz - s)
             ws = _device.ARENA.get('psf_satws', _lib.lib().smx_psf_sat_workspace_bytes(self.nr, m),

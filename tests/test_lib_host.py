@@ -182,3 +182,15 @@ def test_sat_workspace_holds_any_fewer_tables(nr):
     lib = _lib.lib()
     sizes = [int(lib.smx_psf_sat_workspace_bytes(nr, nz)) for nz in range(70)]
     assert sizes == sorted(sizes) and sizes[1] > 0
+
+
+@pytest.mark.parametrize('nr', [2, 1000, 2048, 2049, 4000])
+def test_table_builds_keep_their_scratch_bounded(nr):
+    """The scratch of one build call is at most that of 64 tables' segment sums, or
+    of 8 tables' row sums, which hold every cell."""
+    from scopyon_amd import _psf
+    lib = _lib.lib()
+    ntab = 2 * nr - 1
+    got = int(lib.smx_psf_sat_workspace_bytes(nr, _psf.sat_batch(nr)))
+    assert got <= max(64 << 23, 8 * 8 * ntab * (ntab + 1))
+    assert _psf.sat_batch(nr) == (64 if ntab <= 4096 else 8)
