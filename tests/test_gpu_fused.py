@@ -246,3 +246,27 @@ def test_workspace_across_call_forms(gpu, nfov, n):
             assert torch.equal(call('expected', 32 | warm, ws, phase=False), general)
             assert torch.equal(call('expected', then | warm, ws), listed)
     assert sim.status() == 0
+
+
+def test_heavy_tiles_of_a_large_frame(gpu):
+    """65,536 tiles and more: the counters are scanned by the device scan, and the
+    heavy tiles noted beside it, again in a second step.  Same bits as from fewer,
+    larger tiles, which one workgroup scans."""
+    from scopyon_amd.batched import BatchedSimulator
+    n = 20000
+    rng = numpy.random.RandomState(1)
+    x = rng.uniform(-0.5, 0.5, (2, n)) * numpy.array([[4096], [4112]]) * 1.6e-7
+    x[:, :n // 2] *= 0.03
+    frames = []
+    for side, tiles in ((16, 65792), (32, 16512)):
+        sim = BatchedSimulator(_cfg(), [(4096, 4112)], n, dt=0.033, seed=5, tile_side=side,
+                               keep_photons=True, table_precision='folded')
+        assert sim.n_tiles == tiles
+        sim.set_positions(numpy.zeros(n), x[0], x[1])
+        for step in range(2):
+            sim.splat_detect()
+            frames.append((sim.photons.clone(), sim.adc.clone()))
+        assert sim.status() == 0
+    assert frames[0][0].abs().sum() > 0
+    for photons, adc in frames[1:]:
+        assert torch.equal(photons, frames[0][0]) and torch.equal(adc, frames[0][1])
