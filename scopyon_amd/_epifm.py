@@ -508,8 +508,10 @@ class _EPIFMSimulator:
             p = table[:, 1] / table[:, 1].sum()
             cdf = p.cumsum()
             cdf /= cdf[-1]
-            self._cmos = (_device.upload(table[:, 0], device=self.device),
-                          _device.upload(cdf, device=self.device), len(cdf))
+            # staged: every frame waits for its stream (expose reads the status), so
+            # the copies are complete before another stream can come to use them
+            self._cmos = (_device.stage(table[:, 0], device=self.device),
+                          _device.stage(cdf, device=self.device), len(cdf))
         return self._cmos
 
     def _photon_detector(self, camera, rng, E, adc, gain_map, offset_map, rewind):

@@ -37,11 +37,13 @@ def sat_period(pixel_length):
 
 
 def layout_period(pixel_length):
-    """SAT layout period: the pixel length in cells rounded to an integer.
-    Pixel edges fall floor(ratio) or ceil(ratio) cells apart; with this period
-    the more frequent step keeps a corner's residue, so the corners of
-    neighbouring pixels mostly lie next to each other in memory (runs of ~2.6
-    corners per cache line at 66.4 cells instead of one)."""
+    """Period of the plain SAT layout: the pixel length in cells rounded to an
+    integer.  Pixel edges fall floor(ratio) or ceil(ratio) cells apart; with this
+    period the more frequent step keeps a corner's residue, so the corners of
+    neighbouring pixels mostly lie next to each other in memory.  Phase tables
+    are built from this layout; the splat of pixels that are not whole cells
+    reads the sorted layout instead (PSFTables.places), except from tables too
+    wide for it."""
     ratio = pixel_length / RES
     p = int(round(ratio))
     return p if 2 <= p <= 4096 else 1

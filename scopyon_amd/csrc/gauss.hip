@@ -654,8 +654,9 @@ __global__ void __launch_bounds__(256) gauss_backward_kernel(BwdArgs A) {
 // tile's window of dL/dmu (the tile plus R pixels on every side, zero off
 // the frame) is staged in LDS once; the tile's list (as the forward left it:
 // in emitter order when it was sorted) is filtered to the emitters this tile
-// owns (owner_tile), and each owned emitter is reduced by a 16-lane group
-// exactly as gauss_backward_kernel does, reading LDS instead of the image.
+// owns (owner_tile), and each owned emitter is reduced by four lanes, four
+// window columns a lane, reading LDS instead of the image: the sums of
+// gauss_backward_kernel in the same order.
 // Per tile the dL/dsigma terms are summed in list order with a fixed tree.
 // Workgroups past n_tiles write zero gradients for the emitters no tile owns.
 constexpr int HALO_MAX = TS + 2 * 7;

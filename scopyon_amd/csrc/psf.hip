@@ -101,7 +101,7 @@ __device__ inline double interp_radial(const double* __restrict__ prof, int nr, 
 // radius, interval and offset do not depend on the depth, only the profile
 // value and slope do (LDS).
 // One 2000^2 table 312 us with one wave per row and a serial walk down the
-// columns, 50 us so; 117 tables 14.5 ms before, 1.4 ms so.
+// columns, 66 us so; 117 tables 14.5 ms before, 1.4 ms so.
 constexpr int kCols = 4;              // columns per thread
 constexpr int kSatMax = 1024 * kCols; // widest table of this form
 static_assert(kSatMax == smx::SAT_SORTED_MAX, "sorted tables are built by this form only");
@@ -388,7 +388,8 @@ int sat_build(const double* radial, int nz, int nr, double res, int ntab, smx::S
     const int seg = kSegRows, nseg = (ntab + seg - 1) / seg, nzb = (nz + ZB - 1) / ZB;
     const size_t lds = sizeof(double2) * ZB * (size_t)nr;
     // every block computes the slopes of its profiles, so a block takes whole
-    // rows (64 tables: 168 us, 270 us in panels) unless that leaves CUs idle
+    // rows (64 tables in segments of 32 rows: 168 us, 270 us in panels) unless that
+    // leaves CUs idle
     const int panels = nseg * nzb >= 512 ? 1 : (ntab + kSegThreads - 1) / kSegThreads;
     if (ZB > 1 && 2 * lds <= (64u << 10))
         hipLaunchKernelGGL(sat_segment_kernel<2 * ZB>, dim3(nseg, (nzb + 1) / 2, panels),

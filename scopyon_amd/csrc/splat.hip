@@ -12,10 +12,13 @@
 //
 // Work decomposition: the frame is cut into 32x32-pixel tiles; emitters are
 // binned to the tiles their footprint touches (count -> scan -> fill), each
-// tile's list is sorted by emitter index in LDS (so every pixel adds its
-// contributions in emitter order, like the reference loop, and the result is
-// run-to-run deterministic), then one workgroup per tile accumulates its
-// pixels in LDS.  No float atomics in global memory.
+// tile's list is sorted by emitter index in LDS (so the result is run-to-run
+// deterministic), then one workgroup per tile accumulates its pixels in LDS.
+// With phase or lookup tables every pixel adds its contributions in emitter
+// order, like the reference loop; without (splat_tile_kernel) the first and the
+// second half of the tile's list are added up in emitter order each, then the
+// two sums, which differs from one running sum by rounding of float64.  No
+// float atomics in global memory.
 #include <cstdlib>
 #include <mutex>
 #include <type_traits>
@@ -281,7 +284,7 @@ struct TileArgs {
 //
 // What bounds it is the traffic of the corner loads: the table of a depth key
 // is 32 MB, hardly two emitters of a frame share one, and an emitter needs 32
-// x 32 corners a pixel apart.  In the sorted layout (SatSorted) the corners of
+// x 32 corners a pixel apart.  In the sorted layout (smx_sat_sorted_places) the corners of
 // one footprint row are one run of 32 doubles; the first corner of a row (cell
 // 0, always 0) and the last (cell ntab) would each be a line of their own, so
 // they are read from two vectors beside the table whose rows are runs too.
