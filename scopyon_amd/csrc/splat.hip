@@ -290,7 +290,7 @@ struct TileArgs {
 // they are read from two vectors beside the table whose rows are runs too.
 // 100,000 emitters over 1002 keys on 1024 x 1024 pixels of 66.4 cells:
 // 1.71 ms and 7 GB with corners a tile at a time through LDS from a layout
-// with runs of 2.6 corners, 0.69 ms and 1.5 GB so (0.85 ms with four corner
+// with runs of 2.6 corners, 0.69 ms and 3.3 GB so (0.85 ms with four corner
 // loads per pixel instead of one per corner: the load path's address
 // processing; 0.57 ms when four tables serve every emitter, so what remains is
 // mostly instructions, VALU and LDS, not memory).  Two pieces a quadrant, 51 KB
