@@ -478,8 +478,8 @@ class _EPIFMSimulator:
         # reference order: readout noise (one vector draw), then one uniform
         # per E > 0 pixel inside RandomState.choice (_epifm.py:1449-1454, 393-400);
         # the noise is drawn while the GPU still forms the image
-        noise = (rng.normal(0, c.detector_readout_noise, shape) if c.detector_readout_noise > 0
-                 else None)
+        noise = (None if c.detector_readout_noise <= 0
+                 else rng.normal(0, c.detector_readout_noise, shape))
         count = int((uidx[-1] + flag[-1]).item())
         self._check_splat(rewind)
         if noise is not None:

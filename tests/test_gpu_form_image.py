@@ -314,3 +314,19 @@ def test_failing_frame_leaves_the_generator(gpu, detector, kind):
         assert states() != before
     else:
         assert sim._philox_frame == frame + 1
+
+
+def test_readout_noise_that_is_not_a_number(gpu):
+    """An EMCCD readout noise of NaN is drawn like any other (numpy gives NaN), so
+    that it shows in the counts; the generator advances as for a number."""
+    import scopyon_amd
+    frames, ends = [], []
+    for noise in (100.0, numpy.nan):
+        ov = {'detector': {'type': 'EMCCD', 'image_size': [16, 16], 'readout_noise': noise,
+                           'exposure_time': 0.033}, 'magnification': 100.0}
+        rng = numpy.random.RandomState(3)
+        frames.append(scopyon_amd.form_image(numpy.zeros((1, 2)), config=product_config(ov),
+                                             rng=rng).as_array())
+        ends.append(rng.random_sample())
+    assert numpy.isfinite(frames[0]).all() and ends[0] == ends[1]
+    assert not numpy.array_equal(*frames)
